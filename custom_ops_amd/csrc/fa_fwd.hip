@@ -2021,6 +2021,22 @@ void fa_fwd_kernel_pp(const KParams p) {
   write_rows<D, true, SPLIT>(p, o, lsum[0], mrun[0], ti.b, ti.h, ti.split, qrow, smem + wave * 8192, lane);
 }
 
+// The kernel's parameters, read again from the kernarg segment (scalar loads)
+// where an epilogue needs them: held from the kernel's entry they would spill.
+typedef const __attribute__((address_space(4))) KParams* kernarg_ptr;
+__device__ __forceinline__ kernarg_ptr reload_params() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  kernarg_ptr q = (kernarg_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(q));
+  return q;
+#else
+  return nullptr;   // host pass only: never runs
+#endif
+}
+
+// ── small grids: one key stream per wave ─────────────────────────────────────
+#include "fa_streams.h"
+
 // ── split-KV combine ────────────────────────────────────────────────────────
 struct CParams {
   const uint16_t* o_part;
@@ -2162,6 +2178,65 @@ __global__ __launch_bounds__(kCombineThreads) void fa_combine_kernel(const CPara
   *reinterpret_cast<u32x4*>(dst) = bitcast<u32x4>(__builtin_convertvector(acc, V8));
 }
 
+// More than 16 splits on a small grid (one-wave workgroups): four waves per
+// 64 / (D / 8) rows, each with up to 16 splits' LSEs and partial slices in one
+// round trip and its own running max; the four sums then meet in LDS.
+template <int D, bool BF16>
+__global__ __launch_bounds__(256) void fa_combine_wide_kernel(const CParams p) {
+  typedef typename Elt<BF16>::v8 V8;
+  constexpr int kTPR = D / 8, kRows = 64 / kTPR, kPer = kMaxSplits / 4;
+  __shared__ __align__(16) f32x8 sacc[4][64];
+  __shared__ float sml[4][2][kRows];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane / kTPR, c8 = lane % kTPR;
+  const int64_t row = (int64_t)blockIdx.x * kRows + r;
+  const bool in = row < p.rows;
+  const int per = (p.num_splits + 3) / 4, s0 = wave * per, s1 = min(s0 + per, p.num_splits);
+  const uint32_t sstep = (uint32_t)(p.rows * D * 2), off0 = (uint32_t)((row * D + c8 * 8) * 2);
+  const rsrc_t rp = make_rsrc(p.o_part, p.part_bytes);
+  float l[kPer];
+  u32x4 raw[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {   // past the wave's splits: weight 0, an out-of-range load (0)
+    const bool on = in && s0 + u < s1;
+    l[u] = on ? p.lse_part[(s0 + u) * p.rows + row] : -INFINITY;
+    raw[u] = bload16(rp, on ? off0 + (uint32_t)(s0 + u) * sstep : 0x80000000u);
+  }
+  float mx = -INFINITY;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) mx = fmaxf(mx, l[u]);
+  const float mxc = (mx == -INFINITY) ? 0.f : mx;
+  f32x8 acc = {};
+  float sum = 0.f;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const float w = __builtin_amdgcn_exp2f((l[u] - mxc) * kLog2e);
+    sum += w;
+    acc += w * __builtin_convertvector(bitcast<V8>(raw[u]), f32x8);
+  }
+  sacc[wave][lane] = acc;
+  if (c8 == 0) { sml[wave][0][r] = mx; sml[wave][1][r] = sum; }
+  __syncthreads();
+  if (wave != 0 || !in) return;
+  float m4 = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) m4 = fmaxf(m4, sml[w][0][r]);
+  const float m4c = (m4 == -INFINITY) ? 0.f : m4;
+  f32x8 o = {};
+  float total = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const float e = __builtin_amdgcn_exp2f((sml[w][0][r] - m4c) * kLog2e);
+    total = __builtin_fmaf(e, sml[w][1][r], total);
+    o += e * sacc[w][lane];
+  }
+  o *= (total > 0.f) ? 1.f / total : 0.f;
+  const int64_t bh = row / p.sq;
+  const int m = (int)(row % p.sq), b = (int)(bh / p.h), h = (int)(bh % p.h);
+  uint16_t* dst = p.o + (int64_t)b * p.o_bs + (int64_t)h * p.o_hs + (int64_t)m * p.o_rs + c8 * 8;
+  *reinterpret_cast<u32x4*>(dst) = bitcast<u32x4>(__builtin_convertvector(o, V8));
+}
+
 // ════════════════════════════════════════════════════════════════════════════
 // host side
 // ════════════════════════════════════════════════════════════════════════════
@@ -2263,6 +2338,7 @@ static int env_num_splits() {
 }
 
 struct Plan {
+  int ks;   // streams per workgroup of the key-stream kernel (fa_streams.h): 4 or 8; 0: a tile kernel
   int waves, block_m, num_m, num_n, splits, n_per_split;
   int pack;   // q-heads per workgroup; block_m / pack rows of each
   int head_major;
@@ -2357,6 +2433,82 @@ static int order_head_major(const mi355_fa_params* p, const Plan& pl, int cus,
   return 0;
 }
 
+// ── key-stream plans (fa_streams.h) ──────────────────────────────────────────
+// Modelled launch time of the key-stream kernel with kg streams per workgroup
+// and s splits: n tiles per stream, `blocks` row blocks of 32, R rounds of
+// resident workgroups (two of 4 waves or one of 8 per CU). A stream's tile
+// costs tile + load·R (the streams of a fuller chip share its L2 and MALL
+// bandwidth); each round adds its prologue and merge; kv is K and V's own
+// megabytes; a split launch adds the combine. Least-squares fits on relative
+// error over 370 shapes (row blocks 1 .. 3000, Sk 64 .. 30k, 1 .. 64 splits,
+// inputs not cache-resident), per kg and head dimension, errors 7 - 9 % rms.
+struct StreamCost { float c0, tile, load, round, comb, comb_mb, comb16, kv; };
+constexpr StreamCost kStream4D128 = {3.042f, 0.898f, 0.851f, 2.879f, 2.521f, 0.847f, 0.f, 0.057f};
+constexpr StreamCost kStream8D128 = {1.603f, 1.638f, 0.105f, 5.000f, 2.899f, 0.701f, 0.886f, 0.058f};
+constexpr StreamCost kStream4D64 = {2.229f, 0.734f, 0.492f, 2.750f, 2.672f, 0.805f, 0.340f, 0.029f};
+constexpr StreamCost kStream8D64 = {1.291f, 1.122f, 0.f, 4.175f, 3.315f, 0.450f, 0.849f, 0.038f};
+
+static float stream_cost(const mi355_fa_params* p, int blocks, int kg, int s, int cus) {
+  const StreamCost& c = p->d == 64 ? (kg == 4 ? kStream4D64 : kStream8D64) : (kg == 4 ? kStream4D128 : kStream8D128);
+  const int slots = cus * (8 / kg), n = ceil_div(ceil_div(p->seqlen_k, 32), s * kg);
+  const float R = (float)blocks * (float)s / (float)slots;
+  const float rounds = std::max(1.f, std::ceil(R));
+  float t = c.c0 + (float)n * (c.tile * rounds + c.load * R) + c.round * rounds +
+            c.kv * ((float)p->b * p->h_k * p->seqlen_k * p->d * 4e-6f);
+  if (s > 1)
+    t += c.comb + c.comb_mb * ((float)p->b * p->h * p->seqlen_q * s * p->d * 2e-6f) + (s > 16 ? c.comb16 : 0.f);
+  return t;
+}
+
+// The same shapes' measured times under the tile plan against plan_cost (hot
+// timings on zero masks): a fixed part, a factor, and for masks with unaligned
+// rows the staging pre-pass (a fixed part and its megaentries).
+struct TileCost { float c0, scale, stage, stage_m; };
+constexpr TileCost kTileD128 = {3.68f, 1.10f, 3.54f, 1.73f};
+constexpr TileCost kTileD64 = {3.55f, 1.13f, 3.27f, 0.82f};
+
+// Whether the key-stream kernel runs this call, with how many streams per
+// workgroup (4 or 8; 0: a tile kernel) and splits: where the models put it
+// below the tile plan's `tile_cost`. Over those 370 shapes the choice runs 1.34
+// times as fast as the tile plans alone (geometric mean; the best choice for
+// each shape 1.36), never over 8 % slower. Every stream keeps two tiles. Where
+// several row blocks re-read K and V and the splits are combined the fit is
+// least certain: there it has to win by a fifth. A variant or a split count set
+// by the caller selects among the tile kernels, except waves 1 or 2, which
+// force the streams (4 or 8 per workgroup).
+static int pick_streams(const mi355_fa_params* p, const mi355_fa_variant& v, int cus, bool aligned,
+                        float tile_cost, int* splits) {
+  const mi355_fa_variant none{};
+  const bool forced = v.waves == 1 || v.waves == 2;
+  const int fixed = p->num_splits > 0 ? p->num_splits : env_num_splits();
+  if (!forced && (fixed > 0 || memcmp(&v, &none, sizeof(v)) != 0)) return 0;
+  if (p->seqlen_k < 1) return 0;
+  // bf16 masks are added on the matrix core (see Attn::MMF)
+  if (p->dtype == MI355_FA_BF16 && !(p->scale_softmax < 0.99f)) return 0;
+  const int64_t rows = (int64_t)(p->h / p->h_k) * p->seqlen_q, per = (rows + 31) / 32;
+  const int64_t blocks = (int64_t)p->b * p->h_k * per;
+  if (rows > (1 << 24) || (!forced && blocks > 16 * cus)) return 0;
+  const int ntile = ceil_div(p->seqlen_k, 32);
+  const TileCost& tc = p->d == 64 ? kTileD64 : kTileD128;
+  float limit = tc.c0 + tc.scale * tile_cost;
+  if (!aligned) limit += tc.stage + tc.stage_m * ((float)p->b * p->seqlen_q * p->seqlen_k * 1e-6f);
+  int best = 0;
+  float best_t = 0.f;
+  for (int kg = 4; kg <= 8; kg += 4) {
+    if (forced && kg != 4 * v.waves) continue;
+    int max_s = std::min(kMaxSplits, std::max(1, ntile / (2 * kg)));
+    // more splits than fill the chip twice over only add partials
+    max_s = (int)std::min<int64_t>(max_s, std::max<int64_t>(1, 2 * cus * (8 / kg) / std::max<int64_t>(blocks, 1)));
+    const int lo = forced && fixed > 0 ? std::min(fixed, kMaxSplits) : 1, hi = forced && fixed > 0 ? lo : max_s;
+    for (int s = lo; s <= hi; ++s) {
+      const float t = stream_cost(p, (int)std::min<int64_t>(blocks, 1 << 24), kg, s, cus);
+      if (!forced && t >= (s > 1 && per > 1 ? 0.8f : 1.f) * limit) continue;
+      if (!best || t < best_t) { best = kg; best_t = t; *splits = s; }
+    }
+  }
+  return best;
+}
+
 static Plan make_plan(const mi355_fa_params* p, int cus, bool allow_stage = true) {
   Plan pl{};
   const mi355_fa_variant v = variant_of(p);
@@ -2380,7 +2532,23 @@ static Plan make_plan(const mi355_fa_params* p, int cus, bool allow_stage = true
     }
   }
   if (pl.splits < 1) pl.splits = 1;
+  const bool mask_direct = ((uintptr_t)p->mask & 15) == 0 && (p->mask_batch_stride & 7) == 0 &&
+                           (p->mask_row_stride & 7) == 0;
+  pl.ks = pick_streams(p, v, cus, mask_direct, best, &pl.splits);
   const int s = pl.splits;
+  pl.n_per_split = (s > 1) ? ceil_div(pl.num_n, s) : pl.num_n;
+  if (s > 1) {
+    const size_t rows = (size_t)s * p->b * p->h * p->seqlen_q;
+    pl.o_part_bytes = (rows * p->d * sizeof(uint16_t) + 255) & ~(size_t)255;
+    pl.lse_bytes = (rows * sizeof(float) + 255) & ~(size_t)255;
+  }
+  if (pl.ks) {   // 32 flattened rows per workgroup; the mask is read in place, no live ranges
+    pl.block_m = 32;
+    pl.num_m = ceil_div(p->h / p->h_k * p->seqlen_q, 32);
+    pl.ws_bytes = pl.o_part_bytes + pl.lse_bytes;
+    pl.kv_nt = v.stream < 0 ? 0 : (v.stream > 0 ? 1 : pl.num_m == 1);
+    return pl;
+  }
   pl.block_m = 32 * pl.waves;
   // Workgroup order. Each XCD runs a contiguous range of tile ids with its own
   // L2 (4 MiB, too small to keep a batch's K/V or mask between rounds), so
@@ -2392,11 +2560,7 @@ static Plan make_plan(const mi355_fa_params* p, int cus, bool allow_stage = true
   // short Sq: heads fastest.)
   pl.head_major = order_head_major(p, pl, cus, v);
   pl.num_m = ceil_div(p->seqlen_q, pl.block_m / pl.pack);
-  pl.n_per_split = (s > 1) ? ceil_div(pl.num_n, s) : pl.num_n;
   if (s > 1) {
-    const size_t rows = (size_t)s * p->b * p->h * p->seqlen_q;
-    pl.o_part_bytes = (rows * p->d * sizeof(uint16_t) + 255) & ~(size_t)255;
-    pl.lse_bytes = (rows * sizeof(float) + 255) & ~(size_t)255;
     // one ticket word per row block (batch, head group, m-block)
     const size_t tickets = (size_t)p->b * (p->h / pl.pack) * pl.num_m;
     pl.ticket_bytes = (tickets * 8 + 255) & ~(size_t)255;
@@ -2416,8 +2580,6 @@ static Plan make_plan(const mi355_fa_params* p, int cus, bool allow_stage = true
   // without room for the copy) keep the mask in place: the compiled kernel
   // then reads it through registers, with the map.
   {
-    const bool mask_direct = ((uintptr_t)p->mask & 15) == 0 && (p->mask_batch_stride & 7) == 0 &&
-                             (p->mask_row_stride & 7) == 0;
     // The map also serves 8-wave split launches of aligned masks, whose
     // workgroups would otherwise each scan their rows' dead mask: with the
     // heads and splits that share a row block, a window or causal mask reads
@@ -2578,8 +2740,41 @@ static hipError_t launch_variant(const KParams& kp, const Plan& pl, hipStream_t 
 }
 
 template <int D, bool BF16>
+static hipError_t launch_combine(const CParams& cp, hipStream_t st) {
+  // 256-thread workgroups while they still number >= 1024, else one wave each.
+  constexpr int kRows256 = 256 / (D / 8), kRows64 = 64 / (D / 8);
+  if ((cp.rows + kRows256 - 1) / kRows256 >= 1024) {
+    hipLaunchKernelGGL((fa_combine_kernel<D, BF16, 256>),
+                       dim3((unsigned)((cp.rows + kRows256 - 1) / kRows256)), dim3(256), 0, st, cp);
+  } else if (cp.num_splits > 16 && cp.part_bytes) {
+    hipLaunchKernelGGL((fa_combine_wide_kernel<D, BF16>),
+                       dim3((unsigned)((cp.rows + kRows64 - 1) / kRows64)), dim3(256), 0, st, cp);
+  } else {
+    hipLaunchKernelGGL((fa_combine_kernel<D, BF16, 64>),
+                       dim3((unsigned)((cp.rows + kRows64 - 1) / kRows64)), dim3(64), 0, st, cp);
+  }
+  return hipGetLastError();
+}
+
+template <int D, bool BF16, bool AL>
+static void launch_streams(const KParams& kp, int kg, hipStream_t st) {
+  const dim3 grid(kp.total);
+  switch (kg) {
+    case 4: hipLaunchKernelGGL((fa_fwd_kernel_ks<D, BF16, AL, 4>), grid, dim3(256), 0, st, kp); break;
+    default: hipLaunchKernelGGL((fa_fwd_kernel_ks<D, BF16, AL, 8>), grid, dim3(512), 0, st, kp); break;
+  }
+}
+
+template <int D, bool BF16>
 static hipError_t launch(const KParams& kp_in, const CParams& cp, const Plan& pl, hipStream_t st) {
   KParams kp = kp_in;
+  if (pl.ks) {
+    const bool split = pl.splits > 1;
+    if (kp.mask_direct) launch_streams<D, BF16, true>(kp, pl.ks, st);
+    else launch_streams<D, BF16, false>(kp, pl.ks, st);
+    const hipError_t e = hipGetLastError();
+    return e != hipSuccess || !split ? e : launch_combine<D, BF16>(cp, st);
+  }
   const int lm = pl.live;
   kp.live = pl.num_n >= 4 && (lm == 1 || (lm == 2 && (pl.splits > 1 || !runs_asm_loop<D, BF16>(kp, pl))));
   // the kernels that read the map: the compiled kernel and the ping-pong loop
@@ -2602,16 +2797,7 @@ static hipError_t launch(const KParams& kp_in, const CParams& cp, const Plan& pl
   kf.fuse = kp.fuse && !runs_asm_loop<D, BF16>(kp, pl);
   hipError_t e = launch_variant<D, BF16, true>(kf, pl, st);
   if (e != hipSuccess || kf.fuse) return e;
-  // 256-thread workgroups while they still number >= 1024, else one wave each.
-  constexpr int kRows256 = 256 / (D / 8), kRows64 = 64 / (D / 8);
-  if ((cp.rows + kRows256 - 1) / kRows256 >= 1024) {
-    hipLaunchKernelGGL((fa_combine_kernel<D, BF16, 256>),
-                       dim3((unsigned)((cp.rows + kRows256 - 1) / kRows256)), dim3(256), 0, st, cp);
-  } else {
-    hipLaunchKernelGGL((fa_combine_kernel<D, BF16, 64>),
-                       dim3((unsigned)((cp.rows + kRows64 - 1) / kRows64)), dim3(64), 0, st, cp);
-  }
-  return hipGetLastError();
+  return launch_combine<D, BF16>(cp, st);
 }
 
 }  // namespace mi355fa
@@ -2655,7 +2841,7 @@ static int fwd_impl(const mi355_fa_params* p, void* stream, char* err, size_t er
     return MI355_FA_EDEVICE;
   }
   const Plan pl = make_plan(p, dev.cus, allow_stage);
-  const int64_t total = (int64_t)p->b * (p->h / pl.pack) * pl.num_m * pl.splits;
+  const int64_t total = (int64_t)p->b * (pl.ks ? p->h_k : p->h / pl.pack) * pl.num_m * pl.splits;
   if (total >= (1LL << 24)) {
     set_err(err, errlen, "problem too large: %lld workgroups", (long long)total);
     return MI355_FA_EINVAL;
@@ -2663,7 +2849,7 @@ static int fwd_impl(const mi355_fa_params* p, void* stream, char* err, size_t er
   // Buffer offsets are 32-bit: every per-head / per-batch byte range the kernel
   // addresses (including the rounded-up last row tile) must stay below 2^32.
   {
-    const uint64_t rows_q = (uint64_t)pl.num_m * (pl.block_m / pl.pack), rows_k = (uint64_t)pl.num_n * kBN;
+    const uint64_t rows_q = pl.ks ? (uint64_t)p->seqlen_q : (uint64_t)pl.num_m * (pl.block_m / pl.pack), rows_k = (uint64_t)pl.num_n * kBN;
     const uint64_t lim = 0xffffffffull - 4096;
     const uint64_t need[] = {
         rows_q * (uint64_t)p->q_row_stride * 2, rows_q * (uint64_t)p->o_row_stride * 2,

@@ -51,7 +51,9 @@ enum { MI355_FA_FP16 = 0, MI355_FA_BF16 = 1 };
  * template choices (csrc/fa/fa_fwd_launch.h:262-309).
  */
 typedef struct mi355_fa_variant {
-  int32_t waves;     /* 0 | 4 | 8: waves per workgroup (128 or 256 query rows)         */
+  int32_t waves;     /* 0 | 4 | 8: waves per workgroup (128 or 256 query rows)
+                        | 1 | 2: the key-stream kernel (32 query rows per
+                        workgroup), 4 or 8 key streams                             */
   int32_t pack;      /* 0 | 1 | 2 | 4: GQA q-heads per workgroup (capped by H/Hk)      */
   int32_t order;     /* 0 | 1 heads fastest | 2 m-blocks fastest | 3 heads, then
                         splits fastest (workgroup order)                           */

@@ -186,7 +186,9 @@ struct KParams {
   int n_per_split;   // tiles per split
   int total;         // grid size (workgroups)
   int mask_direct;   // mask rows 16-byte aligned: the mask tile can go by LDS DMA
-  int head_major;    // tile order: 1 heads fastest, 2 heads then splits fastest, 0 m-blocks fastest
+  int head_major;    // tile order: 1 heads fastest, 2 heads then splits fastest, 0 m-blocks fastest,
+                     // 3 / 4 longest first (see tile_index)
+  int sub;           // head groups that run together in order 3
   float scale;       // softmax scale (1/sqrt(d) in the reference op)
   // scale·log2(e) and the rescale slack in score units, as float bits: kernel
   // arguments arrive in SGPRs, which the assembly loops take as scalar operands
@@ -222,6 +224,10 @@ struct KParams {
   const uint16_t* msrc;
   int64_t msrc_bs;
   int msrc_rs, msrc_q;
+  // Shared scan of unsplit ping-pong launches (or null): a word per (batch,
+  // m-block, head group), see share_scan
+  unsigned long long* scan_slots;
+  int scan_group;            // consecutive head groups that share a scan (divides the head groups)
   uint16_t* stage_out;       // the staged copy [B][Sq][stage_rs] (or null)
   int stage_rs;              // ceil(Sk / 8) · 8
 };
@@ -330,7 +336,30 @@ __device__ __forceinline__ TileIdx tile_index(PT& p) {
   int t = xcd_remap(blockIdx.x, p.total);
   const int ng = p.h / p.pack;   // head groups per batch
   int mb, hg;
-  if (p.head_major == 2) {   // (b, m-block, split, head group): every workgroup reading a row block's mask runs together
+  if (p.head_major >= 3) {
+    // Unsplit, longest first: within each XCD's contiguous chunk of ids the
+    // m-blocks run from the last to the first, each for several head groups.
+    // Under a causal mask the live ranges grow with the m-block,
+    // so the short workgroups fill the end of the launch. The chunks are the
+    // plain orders' own: m-blocks dealt out over the XCDs would balance a causal
+    // mask better (GQA [4,16/4,2048,2048] 91 against 102 µs) but cost a dense one
+    // 1.5 % (140.8 against 138.5).
+    const int chunk = p.total / 8, per = ng * p.num_m;
+    const int x = t / chunk, l = t % chunk;
+    if (p.head_major == 3) {            // the chunk holds whole head groups: `sub` at a time, all their m-blocks
+      const int part = p.sub * p.num_m, r = l % part;
+      const int gi = x * (chunk / p.num_m) + l / part * p.sub + r % p.sub;
+      mb = p.num_m - 1 - r / p.sub;
+      hg = gi % ng;
+      ti.b = gi / ng;
+    } else {                            // the chunk holds consecutive m-blocks of all head groups
+      const int cpb = per / chunk, mx = chunk / ng;
+      hg = l % ng;
+      mb = x % cpb * mx + mx - 1 - l / ng;
+      ti.b = x / cpb;
+    }
+    ti.split = 0;
+  } else if (p.head_major == 2) {   // (b, m-block, split, head group): every workgroup reading a row block's mask runs together
     hg = t % ng;  t /= ng;
     ti.split = t % p.num_splits;  t /= p.num_splits;
     mb = t % p.num_m;
@@ -394,12 +423,24 @@ __device__ __forceinline__ void place_wave(TileIdx& ti, const KParams& p, int wa
 // `red` is 4·waves words of LDS that no DMA touches until the final barrier
 // (two sets, used alternately: a set is rewritten two steps after it was read,
 // past the next barrier).
-// Read that way (through a generic pointer) the fields count as divergent, so
-// every field that forms a buffer descriptor or a branch goes through
-// readfirstlane: a descriptor the compiler thinks divergent becomes a
-// waterfall loop (one round trip per load), and a branch it thinks divergent
-// makes every value defined under it divergent too.
-typedef const KParams CKParams;
+// The pointer is a constant-address one, so the fields arrive by scalar loads
+// and count as uniform. (Through a generic pointer each was a vector load with
+// a round trip of its own, and a value the compiler thought divergent.)
+// The kernel's parameters, read again from the kernarg segment (scalar loads)
+// where a probe or an epilogue needs them: held from the kernel's entry they
+// would spill.
+typedef const __attribute__((address_space(4))) KParams* kernarg_ptr;
+__device__ __forceinline__ kernarg_ptr reload_params() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  kernarg_ptr q = (kernarg_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(q));
+  return q;
+#else
+  return nullptr;   // host pass only: never runs
+#endif
+}
+
+typedef const __attribute__((address_space(4))) KParams CKParams;
 // A buffer descriptor whose words are uniform but were computed from values
 // the compiler thinks divergent
 __device__ __forceinline__ rsrc_t make_rsrc_uniform(const void* base, uint32_t bytes) {
@@ -409,30 +450,23 @@ __device__ __forceinline__ rsrc_t make_rsrc_uniform(const void* base, uint32_t b
   return make_rsrc(reinterpret_cast<const void*>(compose_u64(lo, hi)),
                    __builtin_amdgcn_readfirstlane(bytes));
 }
-__device__ __forceinline__ CKParams& kernarg_params(const KParams& pk) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const KParams* kq = (const KParams*)__builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(kq));
-  return *kq;
-#else
-  return pk;   // host pass only: never runs
-#endif
-}
+__device__ __forceinline__ CKParams& kernarg_params(const KParams&) { return *reload_params(); }
 
 // whether the 8 entries of a chunk starting at column c0 hold a visible one
 template <bool BF16>
 __device__ __forceinline__ bool live8(u32x4 v, int c0, int sk) {
   // branch-free (a branch here lets the compiler sink a window load into it,
   // behind the step's wait: a second round trip per step)
-  constexpr uint32_t kNeg = BF16 ? 0xff80u : 0xfc00u;
+  constexpr uint32_t kNeg = BF16 ? 0xff80u : 0xfc00u, kNegPair = kNeg * 0x10001u;
+  // entries from column sk on count as -inf (word i holds entries 2i, 2i + 1)
   const int nv = sk - c0;
-  bool any = false;
+  uint32_t x = 0u;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    any |= (2 * i < nv) & ((v[i] & 0xffffu) != kNeg);
-    any |= (2 * i + 1 < nv) & ((v[i] >> 16) != kNeg);
+    const uint32_t keep = 2 * i + 1 < nv ? ~0u : (2 * i < nv ? 0xffffu : 0u);
+    x |= (v[i] ^ kNegPair) & keep;
   }
-  return any;
+  return x != 0u;
 }
 
 // OR over the wave: within each 16-lane row by DPP, over the four rows by
@@ -482,6 +516,23 @@ __device__ __forceinline__ void wg_or2(uint32_t& a, uint32_t& b, uint32_t* red, 
   b = __builtin_amdgcn_readfirstlane(rb);
 }
 
+// Whether any thread of the workgroup has a / b set: one ballot per wave, one
+// word per wave in LDS (set `set` of two), read by every thread after a barrier
+template <int NT>
+__device__ __forceinline__ void wg_any2(bool& a, bool& b, uint32_t* red, int set) {
+  constexpr int kW = NT / 64;
+  const uint32_t w = (__builtin_amdgcn_ballot_w64(a) ? 1u : 0u) | (__builtin_amdgcn_ballot_w64(b) ? 2u : 0u);
+  uint32_t* r = red + 2 * kW * set;
+  r[threadIdx.x >> 6] = w;
+  __syncthreads();
+  uint32_t x = 0u;
+#pragma unroll
+  for (int i = 0; i < kW; ++i) x |= r[i];
+  x = __builtin_amdgcn_readfirstlane(x);
+  a = (x & 1u) != 0u;
+  b = (x & 2u) != 0u;
+}
+
 // The mask buffer of batch b
 __device__ __forceinline__ rsrc_t mask_rsrc(CKParams& p, int b) {
   return make_rsrc_uniform(p.mask + (int64_t)b * p.m_bs, (uint32_t)p.msq * p.m_rs * 2u);
@@ -489,8 +540,10 @@ __device__ __forceinline__ rsrc_t mask_rsrc(CKParams& p, int b) {
 
 struct LiveProbe { u32x4 l, r; };
 
-template <int NT, bool MAP = false, bool SCAN = true, bool LOCAL = false>
-__device__ __forceinline__ LiveProbe live_probe(const TileIdx& ti, const KParams& pk) {
+// SAMPLE: 8 rows from the first to the last of the workgroup's `rows`, the
+// same for every wave (narrow_to_live's SHARE form).
+template <int NT, bool MAP = false, bool SCAN = true, bool LOCAL = false, bool SAMPLE = false>
+__device__ __forceinline__ LiveProbe live_probe(const TileIdx& ti, const KParams& pk, int rows = 0) {
   CKParams& p = kernarg_params(pk);
   LiveProbe pr{};
   if (!SCAN || !uni(p.live)) return pr;
@@ -499,7 +552,8 @@ __device__ __forceinline__ LiveProbe live_probe(const TileIdx& ti, const KParams
   }
   const rsrc_t rm = mask_rsrc(p, ti.b);
   const int tid = threadIdx.x;
-  const uint32_t rowoff = (uint32_t)(ti.m0 + (tid >> 3)) * (uint32_t)p.m_rs + (uint32_t)(tid & 7) * 8u;
+  const int row = SAMPLE ? ((tid & 63) >> 3) * (max(min(rows, p.sq - ti.m0), 1) - 1) / 7 : tid >> 3;
+  const uint32_t rowoff = (uint32_t)(ti.m0 + row) * (uint32_t)p.m_rs + (uint32_t)(tid & 7) * 8u;
   // LOCAL: the ends of the workgroup's own split range, else of the key axis
   const int t0 = LOCAL ? ti.nb : 0, t1 = LOCAL ? max(ti.ne - 1, 0) : p.num_n - 1;
   pr.l = bload16(rm, (rowoff + (uint32_t)t0 * kBN) * 2u);
@@ -718,15 +772,115 @@ __device__ __forceinline__ bool range_from_map_wave(TileIdx& ti, CKParams& p, in
   return true;
 }
 
+// Shared scan (unsplit ping-pong launches, whose head groups all need the live
+// range of the same rows): instead of each scanning the row block's dead tiles
+// ([4,16,2048,2048] causal: 115 MB of mask per round through the L2s, 17 µs),
+// the sg head groups of a row block that run on one XCD at once divide it:
+// the j-th tests tiles j, j + sg, j + 2·sg, .., publishes the verdicts in its
+// own word, and reads the others' words. That shape: 122 µs with every
+// workgroup scanning, 98-101 shared (131 with no narrowing; all 16 heads, on two
+// XCDs, start apart: 109).
+// A word is a 48-bit launch tag above 16 verdict bits, written and read at
+// device scope (sc1), with one writer, who clears it before it ends: a
+// replayed graph launch, which carries the same tag, finds no word of the
+// replay before. Nothing depends on another workgroup: after a bounded number
+// of polls (head groups that are not running yet) the caller scans by itself.
+// Returns whether the words gave the range [lo, hi] (hi < lo: no visible
+// entry). red: 2·NT/64 words of LDS.
+template <bool BF16, int NT>
+__device__ __forceinline__ bool share_scan(const TileIdx& ti, int rows, int& lo, int& hi, uint32_t* red) {
+  CKParams& p = *reload_params();
+  const int sg = p.scan_group, nn = p.num_n, hg = (ti.h / p.pack) % sg;   // place in the group
+  const int nr = min(rows, p.sq - ti.m0);
+  if (nr <= 0) return false;
+  const int tid = threadIdx.x;
+  const rsrc_t rm = mask_rsrc(p, ti.b);
+  const int cpt = nr * 8;              // 16-byte chunks per tile of these rows
+  constexpr int kJ = 4, kPer = 2;      // chunks per thread and tile (rows <= NT / 2), tiles per step
+  static_assert(NT * kJ >= 256 * 8, "one step covers a tile of 256 rows");
+  uint32_t off[kJ];
+#pragma unroll
+  for (int j = 0; j < kJ; ++j) {
+    const int c = j * NT + tid;
+    off[j] = c < cpt ? ((uint32_t)(ti.m0 + (c >> 3)) * (uint32_t)p.m_rs + (uint32_t)(c & 7) * 8u) * 2u : 0xfffffff0u;
+  }
+  const int c0 = (tid & 7) * 8;
+  uint32_t bits = 0u;                  // bit k: tile hg + k·sg holds a visible entry
+  for (int k = 0; hg + k * sg < nn; k += kPer) {
+    u32x4 v[kPer][kJ];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) {
+        const int t = hg + (k + u) * sg;
+        v[u][j] = bload16(rm, t < nn && off[j] != 0xfffffff0u ? off[j] + (uint32_t)t * (kBN * 2) : 0xfffffff0u);
+      }
+#pragma unroll
+    for (int u = 0; u < kPer; ++u)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) {
+        const int t = hg + (k + u) * sg;
+        const bool in = t < nn && off[j] != 0xfffffff0u;
+        bits |= (in & live8<BF16>(v[u][j], t * kBN + c0, p.sk)) ? 1u << (k + u) : 0u;
+      }
+  }
+  bits = wave_or(bits);
+  if ((tid & 63) == 0) red[tid >> 6] = bits;
+  __syncthreads();
+  unsigned long long* const slots =
+      p.scan_slots + ((int64_t)ti.b * p.num_m + ti.m0 / rows) * (p.h / p.pack) + ti.h / p.pack - hg;
+  if (tid < 64) {
+    uint32_t mine = 0u;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) mine |= red[w];
+    const unsigned long long tag = p.tag << 16;
+    if (tid == 0)
+      __hip_atomic_store(slots + hg, tag | mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    int found = 0, l = 0x7fffffff, h = -1;
+    constexpr int kPolls = 30;         // about 1 µs each
+    for (int it = 0; it < kPolls && !found; ++it) {
+      const unsigned long long w = tid == hg ? tag | mine
+          : tid < sg ? __hip_atomic_load(slots + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : tag;
+      if (__builtin_amdgcn_ballot_w64((w >> 16) != p.tag) == 0) {
+        found = 1;
+        const uint32_t x = (uint32_t)(w & 0xffffu);
+        if (x) { l = tid + __builtin_ctz(x) * sg; h = tid + (31 - __builtin_clz(x)) * sg; }
+      } else {
+        __builtin_amdgcn_s_sleep(16);
+      }
+    }
+    l = wave_min(l);
+    h = wave_max(h);
+    if (tid == 0) { red[NT / 64] = (uint32_t)found; red[NT / 64 + 1] = (uint32_t)l; red[NT / 64 + 2] = (uint32_t)h; }
+  }
+  __syncthreads();
+  const bool ok = __builtin_amdgcn_readfirstlane(red[NT / 64]) != 0u;
+  lo = (int)__builtin_amdgcn_readfirstlane(red[NT / 64 + 1]);
+  hi = (int)__builtin_amdgcn_readfirstlane(red[NT / 64 + 2]);
+  __syncthreads();                     // every wave has read `red`
+  return ok;
+}
+// The workgroup's word, cleared before it ends (see share_scan)
+__device__ __forceinline__ void share_clear(const TileIdx& ti, int rows) {
+  CKParams& p = *reload_params();
+  const int ng = p.h / p.pack;
+  if (threadIdx.x == 0)
+    __hip_atomic_store(p.scan_slots + ((int64_t)ti.b * p.num_m + ti.m0 / rows) * ng + ti.h / p.pack, 0ull,
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // LOCAL (the compiled kernel): a split launch without a map narrows each
 // workgroup's own nominal range [nb, ne) to its live tiles and keeps the
 // nominal partition, so a workgroup scans only its own share of the mask.
 // Scanning the whole axis to re-partition the live range (the assembly
 // loops) reads a sparse mask's dead part once per split and head: a top-left
 // causal [1,16,16,128,32768] took 357 µs that way on 16 splits.
-template <bool BF16, int NT, int BMAX, int J, bool REUSE, bool MAP = false, bool SCAN = true, bool LOCAL = false>
+// SHARE: through share_scan first, when the launch has the words (`shared` is
+// set when the workgroup published its own, which it then has to clear).
+template <bool BF16, int NT, int BMAX, int J, bool REUSE, bool MAP = false, bool SCAN = true, bool LOCAL = false,
+          bool SHARE = false>
 __device__ __forceinline__ bool narrow_to_live(TileIdx& ti, const KParams& pk, int rows, const LiveProbe& pr,
-                                               uint32_t* red) {
+                                               uint32_t* red, bool* shared = nullptr) {
   CKParams& p = kernarg_params(pk);
   if (!uni(p.live)) return false;
   const int nr = uni(min(rows, p.sq - ti.m0));
@@ -744,14 +898,34 @@ __device__ __forceinline__ bool narrow_to_live(TileIdx& ti, const KParams& pk, i
   const int first = LOCAL ? ti.nb : 0, last = LOCAL ? ti.ne - 1 : nn - 1;
   if (LOCAL && first > last) return false;   // an empty share stays empty
   // the probe's verdict: tile first / tile last live in the chunks it read
-  uint32_t lb = ((tid < nr * 8) & live8<BF16>(pr.l, first * kBN + (tid & 7) * 8, p.sk)) ? 1u : 0u;
-  uint32_t rb = ((tid < nr * 8) & live8<BF16>(pr.r, last * kBN + (tid & 7) * 8, p.sk)) ? 1u : 0u;
-  wg_or2<NT>(lb, rb, red, 1);
+  bool lb, rb;
+  if constexpr (SHARE) {
+    // a sample of the rows, the same for every wave: a live entry in it settles
+    // its end without an exchange (a miss only means the scan, which decides)
+    lb = __builtin_amdgcn_ballot_w64(live8<BF16>(pr.l, first * kBN + (tid & 7) * 8, p.sk)) != 0;
+    rb = __builtin_amdgcn_ballot_w64(live8<BF16>(pr.r, last * kBN + (tid & 7) * 8, p.sk)) != 0;
+  } else {
+    lb = (tid < nr * 8) & live8<BF16>(pr.l, first * kBN + (tid & 7) * 8, p.sk);
+    rb = (tid < nr * 8) & live8<BF16>(pr.r, last * kBN + (tid & 7) * 8, p.sk);
+    wg_any2<NT>(lb, rb, red, 1);
+  }
   if (lb && rb) {                          // both ends live: the nominal ranges stand
-    __syncthreads();                       // every wave has read `red` before any DMA lands
+    if constexpr (!SHARE) __syncthreads();   // every wave has read `red` before any DMA lands
     return false;
   }
   int lo = lb ? first : -1, hi = rb ? last : -1;
+  if constexpr (SHARE) {
+    if (p.scan_slots) {
+      *shared = true;
+      int l, h;
+      if (share_scan<BF16, NT>(ti, rows, l, h, red)) {
+        if (h < l) { l = 0; h = -1; }
+        ti.nb = l;
+        ti.ne = h + 1;
+        return true;
+      }
+    }
+  }
   constexpr int kRounds = (8 * BMAX + J * NT - 1) / (J * NT);   // rounds that cover one whole tile
   constexpr int NL = kRounds * J;
   const int cpt = nr * 8;                  // 16-byte chunks per tile of these rows
@@ -881,8 +1055,8 @@ __device__ __forceinline__ int ticket_of(PT& p, const TileIdx& ti) {
   return (ti.b * ng + ti.h / p.pack) * p.num_m + ti.m0 / (BM / p.pack);
 }
 
-template <int D, bool BF16, bool SPLIT>
-__device__ __forceinline__ void write_rows(const KParams& p, const f32x16 (&oacc)[D / 32], float l_run,
+template <int D, bool BF16, bool SPLIT, class P>
+__device__ __forceinline__ void write_rows(P p, const f32x16 (&oacc)[D / 32], float l_run,
                                            float m_run, int b, int h, int split, int qrow, uint8_t* stg,
                                            int lane) {
   constexpr int DB = D / 32;
@@ -910,36 +1084,36 @@ __device__ __forceinline__ void write_rows(const KParams& p, const f32x16 (&oacc
   const int ch = lane % CH, r0 = lane / CH;
   const int row0 = qrow - l32;   // the first of the 32 rows
   if constexpr (!SPLIT) {
-    const rsrc_t ro = make_rsrc(p.o + (int64_t)b * p.o_bs + (int64_t)h * p.o_hs,
-                                (uint32_t)p.sq * p.o_rs * 2u);
+    const rsrc_t ro = make_rsrc(p->o + (int64_t)b * p->o_bs + (int64_t)h * p->o_hs,
+                                (uint32_t)p->sq * p->o_rs * 2u);
 #pragma unroll
     for (int k = 0; k < 32 / RPI; ++k) {
       const int r = r0 + k * RPI;
       const u32x4 v = *reinterpret_cast<const u32x4*>(stg + r * D * 2 + ((ch ^ (r & (CH - 1))) * 16));
       // rows at or past Sq fall outside the buffer and are dropped
-      __builtin_amdgcn_raw_buffer_store_b128(v, ro, (uint32_t)((row0 + r) * p.o_rs + ch * 8) * 2u, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(v, ro, (uint32_t)((row0 + r) * p->o_rs + ch * 8) * 2u, 0, 0);
     }
   } else {
     // partial O normalised by the split's own l, rounded to the input
     // dtype as the reference stores it (fa_fwd_launch.h:289-297)
-    const int64_t bh = (int64_t)b * p.h + h;
-    const int64_t slab = (int64_t)p.b * p.h * p.sq;
-    const int64_t pbase = (int64_t)split * slab + bh * p.sq;
+    const int64_t bh = (int64_t)b * p->h + h;
+    const int64_t slab = (int64_t)p->b * p->h * p->sq;
+    const int64_t pbase = (int64_t)split * slab + bh * p->sq;
     const float lse = (l == 0.f || l != l) ? -INFINITY
-                      : __builtin_fmaf(m_run, p.scale, __builtin_amdgcn_logf(l) * 0.69314718f);
-    if (p.fuse) {
+                      : __builtin_fmaf(m_run, p->scale, __builtin_amdgcn_logf(l) * 0.69314718f);
+    if (p->fuse) {
       // device-scope (sc1) stores: written through to where every XCD reads
       // them, done once this wave's vmcnt drains (the fused tail's release)
-      const rsrc_t rp = make_rsrc(p.o_part, p.part_bytes), rl = make_rsrc(p.lse_part, p.lse_bytes);
+      const rsrc_t rp = make_rsrc(p->o_part, p->part_bytes), rl = make_rsrc(p->lse_part, p->lse_bytes);
 #pragma unroll
       for (int k = 0; k < 32 / RPI; ++k) {
         const int r = r0 + k * RPI;
         const u32x4 v = *reinterpret_cast<const u32x4*>(stg + r * D * 2 + ((ch ^ (r & (CH - 1))) * 16));
-        if (row0 + r < p.sq)
+        if (row0 + r < p->sq)
           __builtin_amdgcn_raw_buffer_store_b128(v, rp, (uint32_t)(((pbase + row0 + r) * D + ch * 8) * 2), 0,
                                                  kCpolSc1);
       }
-      if (g == 0 && qrow < p.sq)
+      if (g == 0 && qrow < p->sq)
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, lse), rl,
                                               (uint32_t)((pbase + qrow) * 4), 0, kCpolSc1);
     } else {
@@ -947,9 +1121,9 @@ __device__ __forceinline__ void write_rows(const KParams& p, const f32x16 (&oacc
       for (int k = 0; k < 32 / RPI; ++k) {
         const int r = r0 + k * RPI;
         const u32x4 v = *reinterpret_cast<const u32x4*>(stg + r * D * 2 + ((ch ^ (r & (CH - 1))) * 16));
-        if (row0 + r < p.sq) *reinterpret_cast<u32x4*>(p.o_part + (pbase + row0 + r) * D + ch * 8) = v;
+        if (row0 + r < p->sq) *reinterpret_cast<u32x4*>(p->o_part + (pbase + row0 + r) * D + ch * 8) = v;
       }
-      if (g == 0 && qrow < p.sq) p.lse_part[pbase + qrow] = lse;
+      if (g == 0 && qrow < p->sq) p->lse_part[pbase + qrow] = lse;
     }
   }
 }
@@ -1481,7 +1655,7 @@ struct Attn {
   }
 
   __device__ __forceinline__ void epilogue(int b, int h, int split, int qrow, uint8_t* stg) {
-    write_rows<D, BF16, SPLIT>(p, oacc, l_run, m_run, b, h, split, qrow, stg, lane);
+    write_rows<D, BF16, SPLIT>(&p, oacc, l_run, m_run, b, h, split, qrow, stg, lane);
   }
 };
 
@@ -1866,7 +2040,7 @@ void fa_fwd_kernel_asm(const KParams p) {
   for (int hh = 0; hh < NH; ++hh) {
     const f32x16 oh[4] = {o[4 * hh], o[4 * hh + 1], o[4 * hh + 2], o[4 * hh + 3]};
     const int qrow = ti.m0 + wave * ROWS + hh * 32 + l32;
-    write_rows<D, BF16, SPLIT>(p, oh, lsum[hh], mrun[hh], ti.b, ti.h, ti.split, qrow,
+    write_rows<D, BF16, SPLIT>(&p, oh, lsum[hh], mrun[hh], ti.b, ti.h, ti.split, qrow,
                                smem + (wave * NH + hh) * 8192, lane);
   }
 }
@@ -1883,6 +2057,10 @@ constexpr int kPpVBase = 3 * kPpKStage;
 constexpr int kPpMBase = 6 * kPpKStage;
 constexpr int kPpLds = kPpMBase + 2 * 32768;    // 160 KiB
 
+// The first tiles' DMA and Q leave before the probe of the mask's two ends is
+// waited for, so that one memory wait covers them all: a dense mask pays for
+// the probe one OR over the workgroup (waited for by itself it cost 2.3 µs of
+// 138 on [4,16,2048,2048], and unsplit launches went without it).
 // MAPPED: the live ranges come from the live-tile map (a launch that has
 // one), else from the probe and scan; the two are separate instances because
 // both in one push the prologue's SGPRs past what the allocator can spill.
@@ -1893,26 +2071,25 @@ void fa_fwd_kernel_pp(const KParams p) {
   constexpr int UPR = D / 8;
   __shared__ __align__(16) uint8_t smem[kPpLds];
   TileIdx ti = tile_index<256>(p);
-  if constexpr (MAPPED) {
-    if (uni(kernarg_params(p).live)) range_from_map_wave(ti, kernarg_params(p), 256 / p.pack);
-  } else {
-    // before the set-up below: its values would be live across the scan, and
-    // the SGPRs the scan needs on top of them would spill
-    const LiveProbe lp = live_probe<512>(ti, p);
-    narrow_to_live<true, 512, 256, 4, false>(ti, p, 256 / p.pack, lp, reinterpret_cast<uint32_t*>(smem + kPpMBase));
-  }
+  const TileIdx tg = ti;   // the workgroup's first head and row
+  bool shared = false;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   place_wave(ti, p, wave, 32);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)smem;
-  const uint16_t* kbase = p.k + (int64_t)ti.b * p.k_bs + (int64_t)ti.hk * p.k_hs;
-  const uint16_t* vbase = p.v + (int64_t)ti.b * p.v_bs + (int64_t)ti.hk * p.v_hs;
-  const uint16_t* mbase = p.mask + (int64_t)ti.b * p.m_bs;
-  const uint32_t kbytes = (uint32_t)p.sk * p.k_rs * 2u, vbytes = (uint32_t)p.sk * p.v_rs * 2u;
-  const uint32_t mbytes = (uint32_t)p.msq * p.m_rs * 2u;
-  const int wa = wave & 3;   // position within the group (group A issues K/V)
-
-  // K/V DMA sources of group-A wave wa, loads i = 0, 1: unit u = wa·64 + lane
+  const int wa = wave & 3;   // position within the group (group A issues K, B V)
+  u32x32 q;
+  {
+    const rsrc_t rq = make_rsrc(p.q + (int64_t)ti.b * p.q_bs + (int64_t)ti.h * p.q_hs, (uint32_t)p.sq * p.q_rs * 2u);
+    const uint32_t qoff = (uint32_t)((ti.m0 + wave * 32 + l32) * p.q_rs + g * 8) * 2u;
+#pragma unroll
+    for (int kd = 0; kd < 8; ++kd) {
+      const u32x4 v = bload16(rq, qoff + kd * 32u);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) q[4 * kd + e] = v[e];
+    }
+  }
+  // K/V DMA sources of wave wa of its group, loads i = 0, 1: unit u = wa·64 + lane
   // of a 16-row slice, row r = u/16 + 16i of the 64-key tile (keys π-permuted
   // per 32); loads 2 and 3 read the same offsets through descriptors 32 rows on
   u32x2 koff, voff;
@@ -1930,6 +2107,68 @@ void fa_fwd_kernel_pp(const KParams p) {
     const int m = i * 8 + lane / 8, slot = lane % 8;
     moff[i] = (uint32_t)((ti.m0 + wave * 32 + m) * p.m_rs + (slot ^ mask_swz(m)) * 8) * 2u;
   }
+  // V rows the last tile's DMA leaves unwritten (Sk % 64) must hold finite
+  // values: zeroed before any wave's DMA can land in the V stages
+  if (p.sk % kBN != 0) {
+    for (int i = tid; i < 3 * kPpKStage / 16; i += 512)
+      reinterpret_cast<u32x4*>(smem + kPpVBase)[i] = u32x4{0u, 0u, 0u, 0u};
+    __syncthreads();
+  }
+  // The loop's entry state: K and mask of tiles n and n + 1 in stages 0 and 1,
+  // V of tile n in stage 0 (waves 0-3 load K, 4-7 V, each its own mask rows).
+  auto first_tiles = [&](int n) {
+    const kernarg_ptr kp = reload_params();
+    auto rsrc = [](const uint16_t* base, uint32_t bytes, uint32_t skip) {
+      return make_rsrc_words(reinterpret_cast<const char*>(base) + skip, bytes > skip ? bytes - skip : 0u);
+    };
+    const bool is_k = wave < 4;
+    const uint32_t rs = (uint32_t)(is_k ? kp->k_rs : kp->v_rs) * 2u, bytes = (uint32_t)kp->sk * rs;
+    const uint16_t* base = is_k ? kp->k + (int64_t)tg.b * kp->k_bs + (int64_t)tg.hk * kp->k_hs
+                                : kp->v + (int64_t)tg.b * kp->v_bs + (int64_t)tg.hk * kp->v_hs;
+    const uint32_t dst = lds0 + (is_k ? 0u : (uint32_t)kPpVBase) + (uint32_t)wa * 1024u;
+    const uint32_t mrow = (uint32_t)kp->m_rs * 2u, mbytes = (uint32_t)kp->msq * mrow;
+    const uint16_t* mbase = kp->mask + (int64_t)tg.b * kp->m_bs;
+    const uint32_t mdst = lds0 + kPpMBase + (uint32_t)(wave * 32 * 128);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const uint32_t row0 = (uint32_t)(n + t) * kBN * rs;
+      if (t == 0 || is_k) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          bload16_lds(rsrc(base, bytes, row0 + (i < 2 ? 0u : 32u * rs)), dst + (uint32_t)(t * kPpKStage + i * 4096),
+                      is_k ? koff[i % 2] : voff[i % 2]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        bload16_lds(rsrc(mbase, mbytes, (uint32_t)(n + t) * kBN * 2u + (i < 2 ? 0u : 16u * mrow)),
+                    mdst + (uint32_t)(t * 32768 + i * 1024), moff[i % 2]);
+    }
+  };
+  auto sgpr = [](uint32_t x) { return __builtin_amdgcn_readfirstlane(x); };
+  // The loop's buffer descriptors for a range that begins at tile n; loads 2
+  // and 3 of each tensor use the second one. They stand at the loop's first
+  // own loads: K and mask tile n + 2, V tile n + 1 (sizes saturating at 0).
+  u32x4 kd0, kd1, vd0, vd1, md0, md1;
+  auto descriptors = [&](int n) {
+    const kernarg_ptr kp = reload_params();
+    auto desc = [&](const uint16_t* base, uint32_t bytes, uint32_t skip) {
+      const uint64_t b = reinterpret_cast<uint64_t>(base) + skip;
+      return u32x4{(uint32_t)sgpr((uint32_t)b), (uint32_t)sgpr((uint32_t)(b >> 32) & 0xffffu),
+                   (uint32_t)sgpr(bytes > skip ? bytes - skip : 0u), (uint32_t)sgpr((uint32_t)kRsrcFlags)};
+    };
+    const uint16_t* kbase = kp->k + (int64_t)tg.b * kp->k_bs + (int64_t)tg.hk * kp->k_hs;
+    const uint16_t* vbase = kp->v + (int64_t)tg.b * kp->v_bs + (int64_t)tg.hk * kp->v_hs;
+    const uint16_t* mbase = kp->mask + (int64_t)tg.b * kp->m_bs;
+    const uint32_t krow = (uint32_t)kp->k_rs * 2u, vrow = (uint32_t)kp->v_rs * 2u, mrow = (uint32_t)kp->m_rs * 2u;
+    const uint32_t kbytes = (uint32_t)kp->sk * krow, vbytes = (uint32_t)kp->sk * vrow;
+    const uint32_t mbytes = (uint32_t)kp->msq * mrow;
+    const uint32_t ksh = (uint32_t)(n + 2) * kBN * krow, vsh = (uint32_t)(n + 1) * kBN * vrow;
+    const uint32_t msh = (uint32_t)(n + 2) * kBN * 2u;
+    kd0 = desc(kbase, kbytes, ksh); kd1 = desc(kbase, kbytes, ksh + 32u * krow);
+    vd0 = desc(vbase, vbytes, vsh); vd1 = desc(vbase, vbytes, vsh + 32u * vrow);
+    md0 = desc(mbase, mbytes, msh); md1 = desc(mbase, mbytes, msh + 16u * mrow);
+  };
+  if constexpr (!MAPPED || !SPLIT) first_tiles(ti.nb);   // (a split's first tile is seldom the nominal one)
   u32x8 krd;
 #pragma unroll
   for (int i = 0; i < 8; ++i) krd[i] = lds0 + (uint32_t)(l32 * UPR + ((2 * i + g) ^ (l32 % UPR))) * 16u;
@@ -1958,52 +2197,56 @@ void fa_fwd_kernel_pp(const KParams p) {
       for (int w = 0; w < 4; ++w) msel[4 * c + w] = (e == 2 * w) ? sb : (e == 2 * w + 1) ? (sb << 16) : 0u;
     }
   }
-  // Q goes straight from HBM into the loop's AGPRs (the loop issues those
-  // loads with its first tiles' DMA): its buffer and this lane's row offset
-  const uint64_t qa = reinterpret_cast<uint64_t>(p.q + (int64_t)ti.b * p.q_bs + (int64_t)ti.h * p.q_hs);
-  uint32_t qoff = (uint32_t)((ti.m0 + wave * 32 + l32) * p.q_rs + g * 8) * 2u;
-  // V rows the last tile's DMA leaves unwritten (Sk % 64) must hold finite
-  // values: zeroed before any wave's DMA can land in the V stages
-  if (p.sk % kBN != 0) {
-    for (int i = tid; i < 3 * kPpKStage / 16; i += 512)
-      reinterpret_cast<u32x4*>(smem + kPpVBase)[i] = u32x4{0u, 0u, 0u, 0u};
-    __syncthreads();
+  if constexpr (MAPPED && !SPLIT) descriptors(ti.nb);
+  if constexpr (MAPPED) {
+    TileIdx tn = tg;
+    if (uni(kernarg_params(p).live)) range_from_map_wave(tn, kernarg_params(p), 256 / reload_params()->pack);
+    const bool again = SPLIT || uni(tn.nb) != ti.nb;
+    ti.nb = tn.nb;
+    ti.ne = tn.ne;
+    if (again) {   // (a wave's DMA goes to parts of the stages that are its own)
+      wait_vmcnt<0>();
+      first_tiles(uni(ti.nb));
+      descriptors(uni(ti.nb));
+    }
+  } else {
+    // (the probe leaves last: its parameter loads then delay nothing)
+    const int rows = 256 / reload_params()->pack;
+    const LiveProbe lp = live_probe<512, false, true, false, !SPLIT>(tg, p, rows);
+    // the scan's words: in a K stage that is not loaded yet (scores of stale
+    // K bytes past Sk are replaced, where stale V bytes would reach O)
+    TileIdx tn = tg;
+    if (narrow_to_live<true, 512, 256, 8, true, false, true, false, !SPLIT>(
+            tn, p, rows, lp, reinterpret_cast<uint32_t*>(smem + 2 * kPpKStage), &shared)) {
+      // the range moved (and every wave's DMA has landed): the first tiles
+      // again if it begins elsewhere
+      const bool again = tn.nb != ti.nb;
+      ti.nb = tn.nb;
+      ti.ne = tn.ne;
+      if (again) {
+        wait_vmcnt<0>();
+        __syncthreads();
+        first_tiles(uni(ti.nb));
+      }
+    }
+    descriptors(uni(ti.nb));   // (held across the scan they would spill)
   }
-  const int nb = ti.nb, ne = ti.ne, cnt = ne - nb;
-
-  const uint32_t ksh = (uint32_t)nb * kBN * (uint32_t)p.k_rs * 2u;
-  const uint32_t vsh = (uint32_t)nb * kBN * (uint32_t)p.v_rs * 2u;
-  const uint32_t msh = (uint32_t)nb * kBN * 2u;
-  const uint64_t ka = reinterpret_cast<uint64_t>(kbase) + ksh;
-  const uint64_t va = reinterpret_cast<uint64_t>(vbase) + vsh;
-  const uint64_t ma = reinterpret_cast<uint64_t>(mbase) + msh;
-  auto sgpr = [](uint32_t x) { return __builtin_amdgcn_readfirstlane(x); };
-  // raw buffer descriptor of `bytes` at `base`, `skip` bytes on (size
-  // saturating at 0); loads 2 and 3 of each tensor use the second one
-  auto desc = [&](uint64_t base, uint32_t bytes, uint32_t skip) {
-    const uint64_t b = base + skip;
-    return u32x4{(uint32_t)sgpr((uint32_t)b), (uint32_t)sgpr((uint32_t)(b >> 32) & 0xffffu),
-                 (uint32_t)sgpr(bytes > skip ? bytes - skip : 0u), (uint32_t)sgpr((uint32_t)kRsrcFlags)};
-  };
-  u32x4 kd0 = desc(ka, kbytes - ksh, 0), kd1 = desc(ka, kbytes - ksh, 32u * p.k_rs * 2u);
-  u32x4 vd0 = desc(va, vbytes - vsh, 0), vd1 = desc(va, vbytes - vsh, 32u * p.v_rs * 2u);
-  u32x4 md0 = desc(ma, mbytes - msh, 0), md1 = desc(ma, mbytes - msh, 16u * p.m_rs * 2u);
-  const uint32_t kstep = sgpr((uint32_t)kBN * p.k_rs * 2u);
-  const uint32_t vstep = sgpr((uint32_t)kBN * p.v_rs * 2u);
+  const kernarg_ptr kp = reload_params();
+  const uint32_t kstep = sgpr((uint32_t)kBN * (uint32_t)kp->k_rs * 2u), vstep = sgpr((uint32_t)kBN * (uint32_t)kp->v_rs * 2u);
+  const int ne = uni(ti.ne), cnt = ne - uni(ti.nb);
   const uint32_t lds_k = sgpr(lds0 + (uint32_t)wa * 1024u);
   const uint32_t lds_v = sgpr(lds0 + (uint32_t)wa * 1024u);   // + kPpVBase in the loop's offsets
   const uint32_t lds_m = sgpr(lds0 + kPpMBase + (uint32_t)(wave * 32 * 128));
-  const uint32_t lim = sgpr((ne == p.num_n && p.sk % kBN) ? (uint32_t)(p.sk % kBN) : 64u);
+  const uint32_t lim = sgpr((ne == kp->num_n && kp->sk % kBN) ? (uint32_t)(kp->sk % kBN) : 64u);
   // host-computed float scalars: kernel arguments, hence SGPRs (a float computed
   // here in VALU and handed to an "s" operand can arrive as a VGPR inside the
   // loop's registers, and an explicit readfirstlane right after the VALU write
   // is a hazard the compiler does not see through inline assembly)
-  const uint32_t c2 = p.c2_bits, slack = p.slack_bits;
+  const uint32_t c2 = kp->c2_bits, slack = kp->slack_bits;
   const uint32_t neginf = sgpr(0xff800000u);
   const uint32_t mclamp = sgpr(0xff7fff7fu);
   const uint32_t ntiles = sgpr((uint32_t)cnt);
   const uint32_t grp = sgpr((uint32_t)(wave >> 2));
-  u32x4 qd = desc(qa, (uint32_t)p.sq * p.q_rs * 2u, 0);
 
   f32x16 o[4];
   float mrun[1], lsum[1];
@@ -2018,20 +2261,13 @@ void fa_fwd_kernel_pp(const KParams p) {
   wait_vmcnt<0>();
   wg_barrier();
   const int qrow = ti.m0 + wave * 32 + l32;
-  write_rows<D, true, SPLIT>(p, o, lsum[0], mrun[0], ti.b, ti.h, ti.split, qrow, smem + wave * 8192, lane);
-}
-
-// The kernel's parameters, read again from the kernarg segment (scalar loads)
-// where an epilogue needs them: held from the kernel's entry they would spill.
-typedef const __attribute__((address_space(4))) KParams* kernarg_ptr;
-__device__ __forceinline__ kernarg_ptr reload_params() {
-#if defined(__HIP_DEVICE_COMPILE__)
-  kernarg_ptr q = (kernarg_ptr)__builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(q));
-  return q;
-#else
-  return nullptr;   // host pass only: never runs
-#endif
+  write_rows<D, true, SPLIT>(reload_params(), o, lsum[0], mrun[0], ti.b, ti.h, ti.split, qrow, smem + wave * 8192, lane);
+  if constexpr (!SPLIT && !MAPPED) {
+    if (shared) {
+      const TileIdx tc = tile_index<256>(*reload_params());
+      share_clear(tc, 256 / reload_params()->pack);
+    }
+  }
 }
 
 // ── small grids: one key stream per wave ─────────────────────────────────────
@@ -2362,6 +2598,9 @@ struct Plan {
   int staged;          // unaligned mask rows copied to an aligned staged mask
   int stage_rs;
   size_t stage_bytes;
+  int sub;             // head groups that run together in order 3
+  int scan_group;      // head groups that share a scan
+  size_t scan_bytes;   // words of the shared scan, after ws_bytes: used when the workspace has room for them
 };
 
 // Tile plan: the workgroup size (4 or 8 waves) and split count with the
@@ -2560,6 +2799,24 @@ static Plan make_plan(const mi355_fa_params* p, int cus, bool allow_stage = true
   // short Sq: heads fastest.)
   pl.head_major = order_head_major(p, pl, cus, v);
   pl.num_m = ceil_div(p->seqlen_q, pl.block_m / pl.pack);
+  // Launches that narrow to live ranges with more workgroups than one round
+  // run the long row blocks first, where the XCD chunks allow it
+  if (s == 1 && v.order == 0 && pl.waves == 8) {
+    const int64_t ng = p->h / pl.pack, total = (int64_t)p->b * ng * pl.num_m, chunk = total / 8;
+    if (total > cus && total % 8 == 0) {
+      if (chunk % pl.num_m == 0 && (pl.head_major == 0 || chunk % (ng * pl.num_m) == 0)) {
+        // as many head groups at a time as fill the XCD's CUs with all their
+        // m-blocks (at least 4, to share the scan): the reuse of m-blocks
+        // fastest; all of a chunk's 8 at once ran [4,16,2048,2048] dense 0.7 %
+        // slower
+        const int64_t nh = chunk / pl.num_m, want = std::max(4, cus / 8 / pl.num_m);
+        pl.sub = (int)nh;
+        while (pl.sub % 2 == 0 && pl.sub / 2 >= want) pl.sub /= 2;
+        pl.head_major = 3;
+      }
+      else if (pl.head_major == 1 && chunk % ng == 0 && (ng * pl.num_m) % chunk == 0) pl.head_major = 4;
+    }
+  }
   if (s > 1) {
     // one ticket word per row block (batch, head group, m-block)
     const size_t tickets = (size_t)p->b * (p->h / pl.pack) * pl.num_m;
@@ -2608,6 +2865,22 @@ static Plan make_plan(const mi355_fa_params* p, int cus, bool allow_stage = true
     pl.stage_bytes = pl.staged ? (((size_t)p->b * p->seqlen_q * pl.stage_rs * 2 + 255) & ~(size_t)255) : 0;
   }
   pl.ws_bytes = pl.o_part_bytes + pl.lse_bytes + pl.ticket_bytes + pl.map_bytes + pl.stage_bytes;
+  // Unsplit ping-pong launches of more than one round whose workgroups probe
+  // and scan (aligned mask rows), in an order that runs a row block's head
+  // groups together (m-blocks fastest, their waits ran [4,16,2048,2048] causal
+  // at 162 µs instead of 102): words for the shared scan, 16 tiles per word
+  {
+    const int ng = p->h / pl.pack;
+    const int64_t total = (int64_t)p->b * ng * pl.num_m;
+    // head groups of a row block that run together
+    const int sg = pl.head_major == 3 && pl.sub < ng ? pl.sub : ng;
+    if (s == 1 && pl.waves == 8 && mask_direct && pl.head_major != 0 && !pl.live_map && pl.live != 0 && pl.loop == 3 && p->d == 128 &&
+        p->dtype == MI355_FA_BF16 && p->scale_softmax < 0.99f && pl.num_n >= 4 && total > cus && ng % sg == 0 &&
+        sg >= 4 && sg <= 64 && pl.num_n <= 16 * sg) {
+      pl.scan_bytes = ((size_t)total * 8 + 255) & ~(size_t)255;
+      pl.scan_group = sg;
+    }
+  }
   // A 4-wave grid that puts at most one workgroup on each CU takes a third K/V
   // stage (112 KiB of LDS at d = 128: one workgroup per CU; cfg4 cold -7 %).
   {
@@ -2776,10 +3049,11 @@ static hipError_t launch(const KParams& kp_in, const CParams& cp, const Plan& pl
     return e != hipSuccess || !split ? e : launch_combine<D, BF16>(cp, st);
   }
   const int lm = pl.live;
-  kp.live = pl.num_n >= 4 && (lm == 1 || (lm == 2 && (pl.splits > 1 || !runs_asm_loop<D, BF16>(kp, pl))));
+  const bool pp = D == 128 && BF16 && pl.loop == 3 && runs_asm_loop<D, BF16>(kp, pl);
+  kp.live = pl.num_n >= 4 && (lm == 1 || (lm == 2 && (pl.splits > 1 || pp || !runs_asm_loop<D, BF16>(kp, pl))));
   // the kernels that read the map: the compiled kernel and the ping-pong loop
   // (the 32- and 64-row loops scan)
-  const bool reads_map = !runs_asm_loop<D, BF16>(kp, pl) || (D == 128 && BF16 && pl.loop == 3);
+  const bool reads_map = !runs_asm_loop<D, BF16>(kp, pl) || pp;
   const bool want_map = kp.live && kp.live_map_out && reads_map;
   if (kp.stage_out || want_map) {
     KParams km = kp;
@@ -2824,7 +3098,8 @@ int mi355_fa_num_splits(const mi355_fa_params* p) {
 
 size_t mi355_fa_workspace_bytes(const mi355_fa_params* p) {
   if (!p || p->d <= 0 || p->seqlen_q <= 0 || p->b <= 0 || p->h <= 0) return 0;
-  return make_plan(p, device_info().cus).ws_bytes;
+  const Plan pl = make_plan(p, device_info().cus);
+  return pl.ws_bytes + pl.scan_bytes;
 }
 
 }  // extern "C"
@@ -2896,6 +3171,7 @@ static int fwd_impl(const mi355_fa_params* p, void* stream, char* err, size_t er
     memcpy(&kp.slack_bits, &slack, 4);
   }
   kp.head_major = pl.head_major;
+  kp.sub = pl.sub;
   kp.mask_direct = (((uintptr_t)p->mask & 15) == 0 && (p->mask_batch_stride & 7) == 0 &&
                     (p->mask_row_stride & 7) == 0) ? 1 : 0;
 
@@ -2916,6 +3192,12 @@ static int fwd_impl(const mi355_fa_params* p, void* stream, char* err, size_t er
     kp.m_bs = (int64_t)p->seqlen_q * pl.stage_rs;
     kp.msq = p->seqlen_q;
     kp.mask_direct = 1;
+  }
+
+  if (pl.scan_bytes && p->workspace && p->workspace_bytes >= pl.ws_bytes + pl.scan_bytes) {
+    kp.scan_slots = (unsigned long long*)((char*)p->workspace + pl.ws_bytes);
+    kp.scan_group = pl.scan_group;
+    kp.tag = next_launch_tag();
   }
 
   CParams cp{};

@@ -1024,17 +1024,16 @@ def pp_dma_items(t_plus2_kstage, t_plus1_vstage, mstage, group_a, parts="kvm"):
 
 
 def gen_pp(bf16: bool = True) -> str:
-    """The ping-pong tile loop: common entry and prologue, then one code path
-    per wave group."""
+    """The ping-pong tile loop: common entry, then one code path per wave group.
+    The first tiles' DMA and Q are the caller's, which can look at the mask
+    while they are in flight."""
     assert bf16
     configure_pp()
     st = Stream()
     L = "fa_pp_%="
-    # Q straight into its AGPRs (row offset in v[TAL], one 16-d step per
-    # immediate offset); these loads land with the prologue's DMA below, so
-    # the workgroup waits once for both
-    for kd in range(KD):
-        st.emit(f"buffer_load_dwordx4 {areg(QA + 4 * kd, 4)}, v{TAL}, s[92:95], 0 offen offset:{kd * 32}")
+    # Q (loaded by the caller into v0-31) to its AGPRs
+    for r in range(32):
+        st.emit(f"v_accvgpr_write_b32 a{QA + r}, v{r}")
     for r in range(64):
         st.emit(f"v_accvgpr_write_b32 a{OA + r}, 0")
     st.emit(f"v_mov_b32 v{MRUN}, %[neginf]")
@@ -1050,23 +1049,9 @@ def gen_pp(bf16: bool = True) -> str:
     st.nop(4)
     st.ready.clear()
 
-    # prologue: K(0), V(0), mask(0) into stage 0, K(1), mask(1) into stage 1
-    # (K by group A, V by group B), all landed before the common barrier
-    st.emit("s_cmp_eq_u32 %[grp], 0")
-    st.emit(f"s_cbranch_scc0 {L}_pb")
-    pa = []
-    for kst in (0, 1):
-        it, _ = pp_dma_items(kst, 0, kst, True, parts="kvm" if kst == 0 else "km")
-        pa += it
-    emit_groups(st, pa)
-    st.emit(f"s_branch {L}_pj")
-    st.emit(f"{L}_pb:")
-    pb = []
-    for kst in (0, 1):
-        it, _ = pp_dma_items(0, 0, kst, False, parts="vm" if kst == 0 else "m")
-        pb += it
-    emit_groups(st, pb)
-    st.emit(f"{L}_pj:")
+    # the caller has issued K(0), V(0), mask(0) into stage 0 and K(1), mask(1)
+    # into stage 1 (K by group A, V by group B), and advanced the descriptors
+    # past them; all of it lands before the common barrier
     st.emit("s_waitcnt vmcnt(0)")
     st.emit("s_barrier")
     st.emit("s_cmp_eq_u32 %[grp], 0")
@@ -1144,18 +1129,18 @@ def pp_group(group_a, L):
 
 def operand_macros_pp():
     outs = [f'"={{{vreg(16 * i, 16)}}}"(o[{i}])' for i in range(4)]
-    outs += [f'"={{v{MRUN}}}"(mrun[0])', f'"={{v{LSUM}}}"(lsum[0])', f'"+{{v{TAL}}}"(qoff)']
+    outs += [f'"={{v{MRUN}}}"(mrun[0])', f'"={{v{LSUM}}}"(lsum[0])']
     # buffer descriptors bound to their SGPR quads (the loop advances them)
     outs += [f'"+{{s[{b}:{b + 3}]}}"({n})' for b, n in ((80, "kd0"), (68, "kd1"), (84, "vd0"), (72, "vd1"),
-                                                         (88, "md0"), (76, "md1"), (92, "qd"))]
-    ins = [f'"{{{vreg(K_OFF, 2)}}}"(koff)', f'"{{{vreg(V_OFF, 2)}}}"(voff)',
+                                                         (88, "md0"), (76, "md1"))]
+    ins = [f'"{{{vreg(0, 32)}}}"(q)', f'"{{{vreg(K_OFF, 2)}}}"(koff)', f'"{{{vreg(V_OFF, 2)}}}"(voff)',
            f'"{{{vreg(M_OFF, 2)}}}"(moff)', f'"{{{vreg(K_RD, 8)}}}"(krd)', f'"{{{vreg(V_RD, 4)}}}"(vrd)',
            f'"{{{vreg(M_RD, 4)}}}"(mrd)', f'"{{{vreg(MSEL, 8)}}}"(msel)']
     ins += [f'[{n}] "s"({n})' for n in ("mclamp", "c2", "slack", "neginf", "lim", "lds_k", "lds_v", "lds_m",
                                          "kstep", "vstep", "ntiles", "grp")]
-    clob = list(range(KWIN, MSEL)) + [MLOG] + [r for r in range(T, NVGPR) if r != TAL]
+    clob = list(range(KWIN, MSEL)) + [MLOG] + list(range(T, NVGPR))
     cl = [f'"v{r}"' for r in clob] + [f'"a{r}"' for r in range(NAGPR)]
-    cl += [f'"s{r}"' for r in range(96, 100)] + ['"m0"', '"vcc"', '"scc"', '"memory"']
+    cl += [f'"s{r}"' for r in range(92, 100)] + ['"m0"', '"vcc"', '"scc"', '"memory"']
     return ["#define MI355_PP_OUTPUTS_BF16 " + ", ".join(outs),
             "#define MI355_PP_INPUTS_BF16 " + ", ".join(ins),
             "#define MI355_PP_CLOBBERS_BF16 " + ", ".join(cl)]

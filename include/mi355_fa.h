@@ -142,9 +142,12 @@ int mi355_fa_fwd_noalloc(const mi355_fa_params* p, void* stream, char* err, size
  * the MI355_FA_NUM_SPLITS override, read once per process, and clamping). */
 int mi355_fa_num_splits(const mi355_fa_params* p);
 
-/* Bytes of workspace mi355_fa_fwd needs for these params (split partials and
+/* Bytes of workspace mi355_fa_fwd uses for these params (split partials and
  * tickets; for masks with unaligned rows the live-tile map and the staged
- * copy; 0 when none of these). */
+ * copy; for large unsplit launches a few kilobytes of words through which
+ * workgroups share their look for the mask's dead tiles; 0 when none of
+ * these). It needs all but the last: with a smaller workspace, or none, such
+ * a launch gives the same result with more mask reads. */
 size_t mi355_fa_workspace_bytes(const mi355_fa_params* p);
 
 /* Pure cost model, exposed for host tests: splits for a problem of

@@ -2899,6 +2899,28 @@ static Plan make_plan(const mi355_fa_params* p, int cus, bool allow_stage = true
   return pl;
 }
 
+// make_plan of everything it depends on, the last one of each thread kept: a
+// call plans once for its workspace's size and its launch.
+static const Plan& plan_for(const mi355_fa_params* p, int cus, bool allow_stage = true) {
+  struct Key {
+    int32_t b, h, h_k, sq, sk, d, dtype, splits, aligned, stage, cus;
+    float scale;
+    mi355_fa_variant v;
+  };
+  static thread_local Key last;
+  static thread_local Plan plan;
+  static thread_local bool have = false;
+  const bool aligned = ((uintptr_t)p->mask & 15) == 0 && (p->mask_batch_stride & 7) == 0 && (p->mask_row_stride & 7) == 0;
+  const Key key = {p->b, p->h, p->h_k, p->seqlen_q, p->seqlen_k, p->d, p->dtype, p->num_splits,
+                   aligned, allow_stage, cus, p->scale_softmax, variant_of(p)};
+  if (!have || memcmp(&key, &last, sizeof(Key)) != 0) {
+    plan = make_plan(p, cus, allow_stage);
+    last = key;
+    have = true;
+  }
+  return plan;
+}
+
 static int validate(const mi355_fa_params* p, char* err, size_t errlen) {
   if (!p) { set_err(err, errlen, "params must not be NULL"); return MI355_FA_EINVAL; }
   if (p->dtype != MI355_FA_FP16 && p->dtype != MI355_FA_BF16) {
@@ -3093,12 +3115,12 @@ int mi355_fa_cost_model_splits(int total_mblocks, int num_n_blocks, int block_m,
 
 int mi355_fa_num_splits(const mi355_fa_params* p) {
   if (!p || p->d <= 0) return 1;
-  return make_plan(p, device_info().cus).splits;
+  return plan_for(p, device_info().cus).splits;
 }
 
 size_t mi355_fa_workspace_bytes(const mi355_fa_params* p) {
   if (!p || p->d <= 0 || p->seqlen_q <= 0 || p->b <= 0 || p->h <= 0) return 0;
-  const Plan pl = make_plan(p, device_info().cus);
+  const Plan& pl = plan_for(p, device_info().cus);
   return pl.ws_bytes + pl.scan_bytes;
 }
 
@@ -3115,7 +3137,7 @@ static int fwd_impl(const mi355_fa_params* p, void* stream, char* err, size_t er
     set_err(err, errlen, "mi355_fa: current HIP device is not gfx950 (MI355X)");
     return MI355_FA_EDEVICE;
   }
-  const Plan pl = make_plan(p, dev.cus, allow_stage);
+  const Plan& pl = plan_for(p, dev.cus, allow_stage);
   const int64_t total = (int64_t)p->b * (pl.ks ? p->h_k : p->h / pl.pack) * pl.num_m * pl.splits;
   if (total >= (1LL << 24)) {
     set_err(err, errlen, "problem too large: %lld workgroups", (long long)total);
@@ -3283,7 +3305,7 @@ extern "C" int mi355_fa_fwd_noalloc(const mi355_fa_params* p, void* stream, char
   bool allow_stage = true;
   if (need > MI355_FA_NOALLOC_SCRATCH_BYTES) {
     allow_stage = false;
-    need = make_plan(p, device_info().cus, false).ws_bytes;
+    need = plan_for(p, device_info().cus, false).ws_bytes;
   }
   if (need > MI355_FA_NOALLOC_SCRATCH_BYTES) {
     set_err(err, errlen,

@@ -4,9 +4,16 @@
 // fa_bindings.cpp:23-43), for PyTorch-ROCm. Built in-tree by
 // custom_ops_amd.build as libmi355_fa_torch.so (linked to libmi355_fa.so next
 // to it); loading it with torch.ops.load_library registers the operator with
-// the reference's schema. This package's own Python shim (fa.py) registers
-// the same operator through torch.library instead, so a process uses one or
-// the other.
+// the reference's schema. This package's own Python side (fa.py) defines the
+// same operator through torch.library instead, so a process uses one or the
+// other.
+//
+// Compiled a second time with MI355_OPS_IMPL_ONLY (libmi355_fa_ops.so), the same
+// function is only the CUDA-key implementation of the operator that fa.py has
+// defined, and reaches the library that fa.py opened through two addresses
+// (mi355_ops_bind). A call of a small problem costs its host work: through the
+// Python implementation and ctypes [1,8,100,200] took 12.5 µs a call, its
+// kernel 7.5.
 //
 // Argument checks: the reference operator's checks, in its order and with its
 // messages (csrc/fa/fa_fwd_op.cu:53-108), so callers see the same
@@ -28,6 +35,14 @@
 #include "mi355_fa.h"
 
 namespace {
+
+#ifdef MI355_OPS_IMPL_ONLY
+decltype(&mi355_fa_fwd) g_fwd = nullptr;
+decltype(&mi355_fa_workspace_bytes) g_workspace_bytes = nullptr;
+#else
+constexpr auto g_fwd = &mi355_fa_fwd;
+constexpr auto g_workspace_bytes = &mi355_fa_workspace_bytes;
+#endif
 
 at::Tensor mha_fwd_with_mask_mi355(const at::Tensor& q, const at::Tensor& k,
                                       const at::Tensor& v, const at::Tensor& mask) {
@@ -85,20 +100,28 @@ at::Tensor mha_fwd_with_mask_mi355(const at::Tensor& q, const at::Tensor& k,
   p.dtype = q.scalar_type() == at::kBFloat16 ? MI355_FA_BF16 : MI355_FA_FP16;
   p.scale_softmax = 1.0f / std::sqrt((float)p.d);
   at::Tensor ws;   // split-KV partials, from the caching allocator
-  if (const size_t n = mi355_fa_workspace_bytes(&p)) {
+  if (const size_t n = g_workspace_bytes(&p)) {
     ws = at::empty({(int64_t)n}, q.options().dtype(at::kByte));
     p.workspace = ws.data_ptr();
     p.workspace_bytes = n;
   }
   char err[512] = {0};
-  const int rc = mi355_fa_fwd(&p, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.device().index()).stream(), err, sizeof err);
+  const int rc = g_fwd(&p, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(q.device().index()).stream(), err, sizeof err);
   TORCH_CHECK(rc == MI355_FA_OK, err);
   return out;
 }
 
 }  // namespace
 
+#ifdef MI355_OPS_IMPL_ONLY
+// The opened library's entry points, set once before the operator is called.
+extern "C" void mi355_ops_bind(void* fwd, void* workspace_bytes) {
+  g_fwd = reinterpret_cast<decltype(g_fwd)>(fwd);
+  g_workspace_bytes = reinterpret_cast<decltype(g_workspace_bytes)>(workspace_bytes);
+}
+#else
 TORCH_LIBRARY_FRAGMENT(recsys_ops, m) {
   m.def("mha_fwd_with_mask(Tensor q, Tensor k, Tensor v, Tensor mask) -> Tensor");
 }
+#endif
 TORCH_LIBRARY_IMPL(recsys_ops, CUDA, m) { m.impl("mha_fwd_with_mask", &mha_fwd_with_mask_mi355); }

@@ -22,10 +22,12 @@ from __future__ import annotations
 
 import ctypes
 import math
+import os
 
 import torch
 
 from . import _lib
+from .build import OPS_PATH
 
 NAMESPACE = "recsys_ops"
 OP_NAME = "mha_fwd_with_mask"
@@ -170,6 +172,29 @@ def _cuda_impl(q, k, v, mask):
 
 _registered = False
 _torch_lib = None
+_ops_lib = None
+
+
+def _bind_native() -> bool:
+    """Load the compiled CUDA-key implementation (csrc/torch_binding.cpp built
+    implementation-only: the checks, workspace and launch of
+    ``mha_fwd_with_mask_hip`` in C++) and hand it the opened library's entry
+    points. False where it was not built against this PyTorch: the Python
+    implementation, which calls the same library, then serves."""
+    global _ops_lib
+    if not os.path.exists(OPS_PATH):
+        return False
+    lib = _lib.load()
+    try:
+        ops = ctypes.CDLL(OPS_PATH)
+    except OSError:
+        return False
+    ops.mi355_ops_bind.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    ops.mi355_ops_bind.restype = None
+    ops.mi355_ops_bind(ctypes.cast(lib.mi355_fa_fwd, ctypes.c_void_p),
+                       ctypes.cast(lib.mi355_fa_workspace_bytes, ctypes.c_void_p))
+    _ops_lib = ops
+    return True
 
 
 def register() -> None:
@@ -179,7 +204,8 @@ def register() -> None:
         return
     lib = torch.library.Library(NAMESPACE, "FRAGMENT")
     lib.define(SCHEMA)
-    lib.impl(OP_NAME, _cuda_impl, "CUDA")
+    if not _bind_native():
+        lib.impl(OP_NAME, _cuda_impl, "CUDA")
     lib.impl(OP_NAME, _cpu_impl, "CPU")
     torch.library.register_fake(f"{NAMESPACE}::{OP_NAME}", lib=lib)(
         lambda q, k, v, mask: torch.empty_like(q))

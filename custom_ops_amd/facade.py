@@ -218,8 +218,12 @@ class RecsysOps:
 
         q [B,H,Sq,d], k/v [B,Hk,Sk,d] (H % Hk == 0), mask [B,1,>=Sq,>=Sk] with
         0 = visible, -inf = blocked, finite = bias. d in {64, 128}."""
-        resolve_backend(backend)
-        self._acquire(OP_GROUPS["mha_fwd_with_mask"])
+        if backend is not None or "CUSTOM_OPS_BACKEND" in os.environ:
+            resolve_backend(backend)
+        # (a slot that is ready is only read: no lock on the per-call path)
+        slot = self._slots["fa"]
+        if not slot.ready:
+            self._acquire("fa")
         return torch.ops.recsys_ops.mha_fwd_with_mask(q, k, v, mask)
 
     def __getattr__(self, name: str):

@@ -1307,13 +1307,13 @@ struct Attn {
   static constexpr bool mdirect = MDIRECT;
   uint32_t k_off[G::kKWaveLoads];
   uint32_t v_off[G::kKWaveLoads];
-  // Mask path. MREG (8 waves, 16-byte aligned rows): each lane loads the 32
-  // mask values of its own row straight into registers. Otherwise the tile
-  // goes through LDS (sM), loaded with 8 lanes per 128-byte row segment:
-  // those grids stream from HBM (4 waves) or read unaligned rows, where the
-  // per-row register loads (32 cache lines per instruction) cost more than
-  // the LDS round trip.
-  static constexpr bool MREG = MDIRECT && WAVES == 8;
+  // Mask path. MREG (8 waves, 16-byte aligned rows, d = 128): each lane loads
+  // the 32 mask values of its own row straight into registers. Otherwise the
+  // tile goes through LDS (sM), loaded with 8 lanes per 128-byte row segment:
+  // those grids stream from HBM (4 waves), read unaligned rows, or have a tile
+  // short enough (d = 64) for the per-row register loads, 32 cache lines per
+  // instruction, to bound it ([4,16,2048,2048] d = 64: 102.6 -> 98.2 µs).
+  static constexpr bool MREG = MDIRECT && WAVES == 8 && D == 128;
   // LDS mask path with bf16 data: the mask can be added on the matrix core
   // (p.mask_mfma): u = A_0·M_0 + A_1·M_1 per 32-key block, where M_c is the
   // 16-key chunk c of the block (keys 16c + 8g .. +7 of the lane's row, the B
@@ -1627,19 +1627,30 @@ struct Attn {
     V8 win[kWin];
 #pragma unroll
     for (int i = 0; i < kWin; ++i) win[i] = rd(i);
-    auto pstep = [&](int j) {
+    // Row sums. 8 waves (two per SIMD): fp32 adds of P before rounding, as the
+    // ping-pong loop sums them (v_dot2 waits on the matrix core, which the
+    // other wave keeps busy); 4 waves: dot products of the rounded P.
+    constexpr bool kSumAdds = WAVES == 8;
+    auto pstep = [&](int j, float& sum) {
       f32x8 pf;
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         pf[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j / 2][(j % 2) * 8 + e], c2, -mlog2));
+      if constexpr (kSumAdds)
+        sum = ((pf[0] + pf[1]) + (pf[2] + pf[3])) + ((pf[4] + pf[5]) + (pf[6] + pf[7]));
       return __builtin_convertvector(pf, V8);
     };
-    V8 pcur = pstep(0);
-    l_run = psum8<BF16>(pcur, l_run);
+    auto add_sum = [&](V8 pv, float sum) {
+      if constexpr (kSumAdds) l_run += sum;
+      else l_run = psum8<BF16>(pv, l_run);
+    };
+    float psum = 0.f;
+    V8 pcur = pstep(0, psum);
+    add_sum(pcur, psum);
 #pragma unroll
     for (int j = 0; j < 2 * NKB; ++j) {
       V8 pnext;
-      if (j + 1 < 2 * NKB) pnext = pstep(j + 1);
+      if (j + 1 < 2 * NKB) pnext = pstep(j + 1, psum);
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
         const int i = j * DB + db;
@@ -1648,7 +1659,7 @@ struct Attn {
         oacc[db] = Elt<BF16>::mfma(a, pcur, oacc[db]);
       }
       if (j + 1 < 2 * NKB) {
-        l_run = psum8<BF16>(pnext, l_run);
+        add_sum(pnext, psum);
         pcur = pnext;
       }
     }

@@ -424,7 +424,8 @@ void fa_fwd_kernel_ks(const KParams p) {
       if (live && (MB == 2 || i > 0)) wait_vmcnt<kLoads>();
       else wait_vmcnt<0>();
       mk.read(mnext, sM + ((i + 1) % MB) * M::kBytes);
-      const bool live_next = M::any(mnext) && i + 1 < cnt;   // (the read has returned)
+      wait_lds();   // with one buffer the next DMA goes where this was read
+      const bool live_next = M::any(mnext) && i + 1 < cnt;
       mk.issue(n + 2 * stride, ntile, ldsM + (uint32_t)((i % MB) * M::kBytes));
       if (live) {
         f32x16 s = a.scores(mraw, sK);

@@ -204,6 +204,9 @@ struct KParams {
   // bf16, scale < 0.99: the compiled kernel's LDS mask path adds the mask on
   // the matrix core (bf16(1/scale) > 1.0078 makes -max_bf16 overflow to -inf)
   int mask_mfma;
+  // the staged mask copy holds no +inf or NaN (mask_finite): no such entry can
+  // stand behind Sk in a tile, but for LDS bytes that nothing has written
+  int mask_clean;
   // K/V tiles are read by exactly one workgroup each: the compiled kernel
   // streams them with the non-temporal hint
   int kv_nt;
@@ -281,6 +284,20 @@ __device__ __forceinline__ f32x16 mask_to_f32(u32x4 lo, u32x4 hi) {
 #pragma unroll
   for (int i = 0; i < 8; ++i) { r[i] = a[i]; r[8 + i] = b[i]; }
   return r;
+}
+
+// Mask entries for the matrix core, where a zero of the selector meets every
+// entry of the row: +inf and positive NaN to max_bf16 (negative ones are clamped
+// with -inf). In the tile that reaches past Sk the entries behind Sk are
+// anything at all: the caller's pad columns, the next row, or what
+// out-of-range DMA lanes left in the LDS. (Their scores are replaced by -inf; a
+// visible +inf or NaN still makes its row NaN, as max_bf16·(1/scale) is +inf.)
+__device__ __forceinline__ u32x4 mask_finite(u32x4 x) {
+  typedef short s2 __attribute__((ext_vector_type(2)));
+  const s2 lim = {0x7f7f, 0x7f7f};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) x[j] = bitcast<uint32_t>(__builtin_elementwise_min(bitcast<s2>(x[j]), lim));
+  return x;
 }
 
 // max / sum with the lane 32 apart (the other half of the same query row)
@@ -725,6 +742,7 @@ __global__ __launch_bounds__(256) void mask_stage_kernel(KParams p) {
         if (c0 + j >= sk)
           w[j >> 1] = (j & 1) ? ((w[j >> 1] & 0xffffu) | (kNeg << 16)) : ((w[j >> 1] & 0xffff0000u) | kNeg);
     }
+    if (BF16 && p.mask_clean) w = mask_finite(w);
     const bool live = !((w[0] == kNegPair) & (w[1] == kNegPair) & (w[2] == kNegPair) & (w[3] == kNegPair));
     if (live) mine |= 1u << (lane >> 3);
     if (p.stage_out)
@@ -1505,13 +1523,23 @@ struct Attn {
   static constexpr int kWin = 2;
   typedef f32x16 Scores[NKB];
 
-  __device__ __forceinline__ void mask_init(const uint16_t* sM) { mask_init(sM, s); }
-  __device__ __forceinline__ void mask_init(const uint16_t* sM, Scores& sc) {
+  __device__ __forceinline__ void mask_init(int n, uint16_t* sM) { mask_init(n, sM, s); }
+  __device__ __forceinline__ void mask_init(int n, uint16_t* sM, Scores& sc) {
     const uint8_t* mb = reinterpret_cast<const uint8_t*>(sM);
     if constexpr (MMF) {
       if (mmfma) {
         typedef unsigned short us2 __attribute__((ext_vector_type(2)));
         const us2 lim = {0xff7fu, 0xff7fu};   // -max_bf16: -inf (0xff80) and above clamp to it
+        // The tile that reaches past Sk: the wave's rows made finite in LDS, each
+        // lane the units it loaded. (On the registers below it cost every tile:
+        // 29.1 against 28.5 µs on [2,16/4,1024,1024].)
+        if (__builtin_expect((n + 1) * kBN > p.sk, 0)) {
+#pragma unroll
+          for (int i = 0; i < G::kMWaveLoads; ++i) {
+            u32x4* x = reinterpret_cast<u32x4*>(sM + ((tid & ~63) * G::kMWaveLoads + i * 64 + lane) * 8);
+            *x = mask_finite(*x);
+          }
+        }
 #pragma unroll
         for (int b = 0; b < NKB; ++b) {
 #pragma unroll
@@ -1783,7 +1811,7 @@ void fa_fwd_kernel(const KParams p) {
   }
   if (cnt > 0) {
     a.commit_m(sM);
-    a.mask_init(sM);
+    a.mask_init(nb, sM);
   }
 
   // Loads of one iteration, in issue order: the mask's, then K's, then V's.
@@ -1820,13 +1848,13 @@ void fa_fwd_kernel(const KParams p) {
       // loads, and with them for the K/V DMAs issued later). Kept inside this
       // iteration: hoisted past the next barrier it would hold mask(n + 1)'s
       // registers across mask(n + 2)'s loads.
-      a.mask_init(sM);
+      a.mask_init(n + 1, sM);
       __builtin_amdgcn_sched_barrier(0);
     } else if (more) {
       if (far) wait_vmcnt<kKVLoads>();
       else wait_vmcnt<0>();
       a.commit_m(sM);
-      a.mask_init(sM);
+      a.mask_init(n + 1, sM);
     }
   };
   // Unrolled by NST so every stage index is a compile-time constant; the
@@ -2119,9 +2147,11 @@ void fa_fwd_kernel_pp(const KParams p) {
     moff[i] = (uint32_t)((ti.m0 + wave * 32 + m) * p.m_rs + (slot ^ mask_swz(m)) * 8) * 2u;
   }
   // V rows the last tile's DMA leaves unwritten (Sk % 64) must hold finite
-  // values: zeroed before any wave's DMA can land in the V stages
+  // values: zeroed before any wave's DMA can land in the V stages. The same for
+  // the mask's last row, whose units past the mask's end stay unwritten.
   if (p.sk % kBN != 0) {
-    for (int i = tid; i < 3 * kPpKStage / 16; i += 512)
+    const int end = tg.m0 + 256 / p.pack >= p.sq ? kPpLds : kPpMBase;
+    for (int i = tid; i < (end - kPpVBase) / 16; i += 512)
       reinterpret_cast<u32x4*>(smem + kPpVBase)[i] = u32x4{0u, 0u, 0u, 0u};
     __syncthreads();
   }
@@ -2257,7 +2287,8 @@ void fa_fwd_kernel_pp(const KParams p) {
   const uint32_t neginf = sgpr(0xff800000u);
   const uint32_t mclamp = sgpr(0xff7fff7fu);
   const uint32_t ntiles = sgpr((uint32_t)cnt);
-  const uint32_t grp = sgpr((uint32_t)(wave >> 2));
+  // bit 0: the wave's group; bit 1: the last tile's mask needs mask_finite
+  const uint32_t grp = sgpr((uint32_t)(wave >> 2) | (kp->sk % kBN && !kp->mask_clean ? 2u : 0u));
 
   f32x16 o[4];
   float mrun[1], lsum[1];
@@ -3225,6 +3256,7 @@ static int fwd_impl(const mi355_fa_params* p, void* stream, char* err, size_t er
     kp.m_bs = (int64_t)p->seqlen_q * pl.stage_rs;
     kp.msq = p->seqlen_q;
     kp.mask_direct = 1;
+    kp.mask_clean = kp.mask_mfma;
   }
 
   if (pl.scan_bytes && p->workspace && p->workspace_bytes >= pl.ws_bytes + pl.scan_bytes) {

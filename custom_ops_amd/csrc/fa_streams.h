@@ -59,8 +59,8 @@ template <int D, bool BF16> struct StreamRows {
     }
   }
 
-  // u = mask·(1/scale) + K·Qᵀ of one 32-key tile
-  __device__ __forceinline__ f32x16 scores(const u32x4 (&mask)[2], const uint8_t* sK) {
+  // u = mask·(1/scale) + K·Qᵀ of one 32-key tile (left: keys from its first to Sk)
+  __device__ __forceinline__ f32x16 scores(const u32x4 (&mask)[2], int left, const uint8_t* sK) {
     // all K reads at once (two in flight, as the compiler would order them,
     // leave the matrix core waiting for the LDS)
     V8 a[KD];
@@ -74,6 +74,7 @@ template <int D, bool BF16> struct StreamRows {
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         u32x4 x = mask[c];
+        if (left < kTS) x = mask_finite(x);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           x[j] = bitcast<uint32_t>(__builtin_elementwise_min(bitcast<us2>(x[j]), lim));
@@ -428,10 +429,11 @@ void fa_fwd_kernel_ks(const KParams p) {
       const bool live_next = M::any(mnext) && i + 1 < cnt;
       mk.issue(n + 2 * stride, ntile, ldsM + (uint32_t)((i % MB) * M::kBytes));
       if (live) {
-        f32x16 s = a.scores(mraw, sK);
+        const int left = p.sk - n * kTS;
+        f32x16 s = a.scores(mraw, left, sK);
         wait_lds();
         if (live_next) issue_k(n + stride);
-        const bool some = a.rescale(s, p.sk - n * kTS, g);
+        const bool some = a.rescale(s, left, g);
         V8 pj[2];
         if (some) {
 #pragma unroll

@@ -127,6 +127,7 @@ class Stream:
 
     def __init__(self):
         self.lines = []
+        self.far = []       # rarely executed blocks, placed behind the code
         self.pos = 0
         self.ready = {}     # reg -> (position it was written, min distance for VALU readers)
 
@@ -497,7 +498,21 @@ def mask_add_valus(bf16, s_next, mstage_off):
     return out
 
 
-def mask_mfma_items(s_next, mstage_off):
+def mask_tail_item(st, label, regs, needs, left):
+    """Mask entries past Sk in the last tile (s92 == left, Sk % 64 != 0) are
+    anything at all (the caller's pad columns, what out-of-range DMA lanes left
+    in the LDS): +inf and positive NaN to max_bf16, as a zero of the selector
+    times them would be NaN in every key of the row. Their own scores are
+    replaced by -inf (tail_item). The block stands behind the loop (st.far)."""
+    st.far += [f"{label}_far:", "s_cmp_eq_u32 %[lim], 64", f"s_cbranch_scc1 {label}_back",
+               "s_mov_b32 s93, 0x7f7f7f7f"]
+    st.far += [f"v_pk_min_i16 v{r}, v{r}, s93" for r in regs]
+    st.far += [f"s_nop {W_VALU_MFMA}", f"s_branch {label}_back"]
+    return {"kind": "raw", "needs": needs, "lines":
+            [f"s_cmp_eq_u32 s92, {left}", f"s_cbranch_scc1 {label}_far", f"{label}_back:"]}
+
+
+def mask_mfma_items(st, s_next, mstage_off, label, left):
     """bf16: u += mask·(1/scale) on the matrix core. The mask chunk of 16 keys
     (half h, block b, chunk c: keys 32b + 16c + 8g .. +7 of this lane's row) is
     the B operand as it sits in LDS; the A operand A_c (v[MSEL + 4c ..]) holds
@@ -505,7 +520,8 @@ def mask_mfma_items(s_next, mstage_off):
     16c + k of its k index, else 0, so the MFMA adds mask·(1/scale) to exactly
     the matching score. -inf is first clamped to -max_bf16 (v_pk_min_u16; 0 ×
     -inf would be NaN); -max·(1/scale) overflows fp32 back to -inf because
-    bf16(1/scale) > 1.0078 (checked on the host). Returns (mfmas, valus)."""
+    bf16(1/scale) > 1.0078 (checked on the host). label, left: see
+    mask_tail_item. Returns (mfmas, valus), 5 valus per chunk."""
     mf, va = [], []
     slots = MSLOTS
     for idx, (h, b, c) in enumerate([(h, b, c) for h in range(NH) for b in range(2) for c in range(2)]):
@@ -518,6 +534,7 @@ def mask_mfma_items(s_next, mstage_off):
             it = valu(f"v_pk_min_u16 v{w + r}, v{w + r}, %[mclamp]", [w + r], [w + r], needs=[ld])
             it["tag"] = tag
             va.append(it)
+        va.append(dict(mask_tail_item(st, f"{label}{idx}", vrange(w, 4), [ld], left), tag=tag))
         dst = S(s_next, h, b, 0)
         mf.append({"kind": "mfma", "needs": [ld], "deps": (tag,),   # the slot stays held until here
                    "text": f"v_mfma_f32_32x32x16_bf16 {vreg(dst, 16)}, {vreg(MSEL + 4 * c, 4)}, "
@@ -728,7 +745,7 @@ def gen(bf16: bool, nh: int = 2) -> str:
     st.emit("s_barrier")
     Phase(st).run(qk_mfmas(bf16, K_LDS, 0), [])
     if bf16:
-        mm, clamps = mask_mfma_items(0, M_LDS)
+        mm, clamps = mask_mfma_items(st, 0, M_LDS, f"{L}_m0", 1)
         Phase(st).run(mm, clamps)
         st.nop(W_MFMA_VALU)
         Phase(st).run([], [tail_item(f"{L}_t0", 0)] + max_valus(0))
@@ -761,7 +778,7 @@ def gen(bf16: bool, nh: int = 2) -> str:
             balanced_body(st, qk, pv, ex, others, nxt, lab)
             return
         if bf16:
-            mm, clamps = mask_mfma_items(nxt, M_LDS + nxt * MSTAGE)
+            mm, clamps = mask_mfma_items(st, nxt, M_LDS + nxt * MSTAGE, f"{lab}_m", 2)
             mfy = []
             for i, m in enumerate(pv):
                 mfy.append(m)
@@ -799,10 +816,10 @@ def gen(bf16: bool, nh: int = 2) -> str:
         before PV step j), the tail and row max of n+1 once S(n+1) is final.
         The tile's DMA issues under the first half of the MFMAs."""
         p = 1 - nxt
-        mm, clamps = mask_mfma_items(nxt, M_LDS + nxt * MSTAGE)
+        mm, clamps = mask_mfma_items(st, nxt, M_LDS + nxt * MSTAGE, f"{lab}_m", 2)
         mf = qk[:16] + mm + qk[16:] + pv
         for idx in range(len(mm)):
-            for it in clamps[4 * idx:4 * idx + 4]:
+            for it in clamps[5 * idx:5 * idx + 5]:
                 it["deadline"] = 16 + idx
         cv = cvt_valus(bf16, p)
         chain = []
@@ -842,7 +859,11 @@ def gen(bf16: bool, nh: int = 2) -> str:
     for r in range(64 * NH):
         st.emit(f"v_accvgpr_read_b32 v{r}, a{OA + r}")
     st.nop(2)
-    return "\n".join(st.lines)
+    return "\n".join(st.lines + far_blocks(st.far, f"{L}_done"))
+
+
+def far_blocks(far, done):
+    return [f"s_branch {done}"] + far + [f"{done}:"] if far else []
 
 
 # ── ping-pong form (bf16, 8 waves of 32 rows) ────────────────────────────────
@@ -933,7 +954,7 @@ PP_MCHUNKS = [(0, 0), (1, 0), (0, 1), (1, 1)]   # (block b, chunk c), issue orde
 
 def pp_mask_preread(mstage):
     """mask(t+1) chunks read into the V window and clamped (-inf -> -max_bf16);
-    the M phase's mask MFMAs take them from there."""
+    the M phase's mask MFMAs take them from there (the last tile's: pp_last_mask)."""
     out = []
     for idx, (b, c) in enumerate(PP_MCHUNKS):
         w = VWIN + 4 * idx
@@ -941,6 +962,20 @@ def pp_mask_preread(mstage):
         for r in range(4):
             out.append(valu(f"v_pk_min_u16 v{w + r}, v{w + r}, %[mclamp]", [w + r], [w + r], needs=[ld]))
     return out
+
+
+def pp_last_mask(label, back, final=None):
+    """Reached when the tile about to be scored is the last (or, with final, when
+    none is left: on to that label). If it reaches past Sk and the mask is not a
+    staged copy without +inf and NaN (bit 1 of grp), its chunks in the V window
+    are made finite, as in mask_tail_item. Only the loop's own end test leads
+    here: a test of its own in every tile cost the loop 1 %, and going through
+    here a 30 µs launch 1.2 µs ([2,16/4,1000,4099] on 2 splits, staged)."""
+    test = ["s_cmp_eq_u32 s92, 0", f"s_cbranch_scc1 {final}"] if final else []
+    return [f"{label}:"] + test + \
+        ["s_bitcmp1_b32 %[grp], 1", f"s_cbranch_scc0 {back}", "s_mov_b32 s93, 0x7f7f7f7f"] + \
+        [f"v_pk_min_i16 v{r}, v{r}, s93" for r in range(VWIN, VWIN + 4 * len(PP_MCHUNKS))] + \
+        [f"s_nop {W_VALU_MFMA}", f"s_branch {back}"]
 
 
 def pp_mask_mfmas(sbuf):
@@ -1054,12 +1089,13 @@ def gen_pp(bf16: bool = True) -> str:
     # past them; all of it lands before the common barrier
     st.emit("s_waitcnt vmcnt(0)")
     st.emit("s_barrier")
-    st.emit("s_cmp_eq_u32 %[grp], 0")
-    st.emit(f"s_cbranch_scc0 {L}_gb")
+    st.emit("s_bitcmp1_b32 %[grp], 0")
+    st.emit(f"s_cbranch_scc1 {L}_gb")
     head = list(st.lines)
-    ga = pp_group(True, L + "_a")
-    gb = pp_group(False, L + "_b")
-    return "\n".join(head + ga + [f"s_branch {L}_end", f"{L}_gb:"] + gb + [f"{L}_end:"] + pp_tail())
+    ga, fa = pp_group(True, L + "_a")
+    gb, fb = pp_group(False, L + "_b")
+    return "\n".join(head + ga + [f"s_branch {L}_end", f"{L}_gb:"] + gb + [f"{L}_end:"] + pp_tail()
+                     + far_blocks(fa + fb, f"{L}_done"))
 
 
 def pp_tail():
@@ -1105,18 +1141,27 @@ def pp_group(group_a, L):
         Phase(st, PP_MAXQ).run([], vy)
         st.emit("s_barrier")
 
+    def end_test(t, r):
+        """s92 tiles are left after the one whose V phase has just run"""
+        st.emit("s_cmp_le_u32 s92, 1")
+        st.emit(f"s_cbranch_scc1 {L}_n{r}")
+        st.emit(f"{L}_c{r}:")
+        st.far.extend(pp_last_mask(f"{L}_n{r}", f"{L}_c{r}", f"{L}_f{t}"))
+
+    st.emit("s_cmp_eq_u32 s92, 0")
+    st.emit(f"s_cbranch_scc1 {L}_n")
+    st.emit(f"{L}_c:")
+    st.far.extend(pp_last_mask(f"{L}_n", f"{L}_c"))
     m_phase(0, True, False, None)
     v_phase(0, f"{L}_v0")
-    st.emit("s_cmp_eq_u32 s92, 0")
-    st.emit(f"s_cbranch_scc1 {L}_f0")
+    end_test(0, 0)
     st.emit(f"{L}_loop:")
     for r in range(1, 7):
         t = r % 6
         m_phase(t, False, False, True)
         st.emit("s_sub_u32 s92, s92, 1")
         v_phase(t, f"{L}_v{r}")
-        st.emit("s_cmp_eq_u32 s92, 0")
-        st.emit(f"s_cbranch_scc1 {L}_f{t}")
+        end_test(t, r)
     st.emit(f"s_branch {L}_loop")
     for t in range(6):
         st.emit(f"{L}_f{t}:")
@@ -1124,7 +1169,7 @@ def pp_group(group_a, L):
         st.emit(f"s_branch {L}_x")
     st.emit(f"{L}_x:")
     st.emit("s_waitcnt vmcnt(0)")
-    return st.lines
+    return st.lines, st.far
 
 
 def operand_macros_pp():

@@ -1655,30 +1655,19 @@ struct Attn {
     V8 win[kWin];
 #pragma unroll
     for (int i = 0; i < kWin; ++i) win[i] = rd(i);
-    // Row sums. 8 waves (two per SIMD): fp32 adds of P before rounding, as the
-    // ping-pong loop sums them (v_dot2 waits on the matrix core, which the
-    // other wave keeps busy); 4 waves: dot products of the rounded P.
-    constexpr bool kSumAdds = WAVES == 8;
-    auto pstep = [&](int j, float& sum) {
+    auto pstep = [&](int j) {
       f32x8 pf;
 #pragma unroll
       for (int e = 0; e < 8; ++e)
         pf[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j / 2][(j % 2) * 8 + e], c2, -mlog2));
-      if constexpr (kSumAdds)
-        sum = ((pf[0] + pf[1]) + (pf[2] + pf[3])) + ((pf[4] + pf[5]) + (pf[6] + pf[7]));
       return __builtin_convertvector(pf, V8);
     };
-    auto add_sum = [&](V8 pv, float sum) {
-      if constexpr (kSumAdds) l_run += sum;
-      else l_run = psum8<BF16>(pv, l_run);
-    };
-    float psum = 0.f;
-    V8 pcur = pstep(0, psum);
-    add_sum(pcur, psum);
+    V8 pcur = pstep(0);
+    l_run = psum8<BF16>(pcur, l_run);
 #pragma unroll
     for (int j = 0; j < 2 * NKB; ++j) {
       V8 pnext;
-      if (j + 1 < 2 * NKB) pnext = pstep(j + 1, psum);
+      if (j + 1 < 2 * NKB) pnext = pstep(j + 1);
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
         const int i = j * DB + db;
@@ -1687,7 +1676,7 @@ struct Attn {
         oacc[db] = Elt<BF16>::mfma(a, pcur, oacc[db]);
       }
       if (j + 1 < 2 * NKB) {
-        add_sum(pnext, psum);
+        l_run = psum8<BF16>(pnext, l_run);
         pcur = pnext;
       }
     }

@@ -2737,6 +2737,15 @@ struct TileCost { float c0, scale, stage, stage_m; };
 constexpr TileCost kTileD128 = {3.68f, 1.10f, 3.54f, 1.73f};
 constexpr TileCost kTileD64 = {3.55f, 1.13f, 3.27f, 0.82f};
 
+// Whether bf16(1/scale), the weight of a mask added on the matrix core, is 1/scale
+// (as at d = 64 with the operator's scale: 8)
+static bool exact_mask_weight(float scale) {
+  const float w = 1.f / scale;
+  uint32_t bits;
+  memcpy(&bits, &w, 4);
+  return (bits & 0xffffu) == 0 && w * scale == 1.f;
+}
+
 // Whether the key-stream kernel runs this call, with how many streams per
 // workgroup (4 or 8; 0: a tile kernel) and splits: where the models put it
 // below the tile plan's `tile_cost`. Over those 370 shapes the choice runs 1.34
@@ -2747,14 +2756,19 @@ constexpr TileCost kTileD64 = {3.55f, 1.13f, 3.27f, 0.82f};
 // by the caller selects among the tile kernels, except waves 1 or 2, which
 // force the streams (4 or 8 per workgroup).
 static int pick_streams(const mi355_fa_params* p, const mi355_fa_variant& v, int cus, bool aligned,
-                        float tile_cost, int* splits) {
+                        int tile_waves, float tile_cost, int* splits) {
   const mi355_fa_variant none{};
   const bool forced = v.waves == 1 || v.waves == 2;
   const int fixed = p->num_splits > 0 ? p->num_splits : env_num_splits();
   if (!forced && (fixed > 0 || memcmp(&v, &none, sizeof(v)) != 0)) return 0;
   if (p->seqlen_k < 1) return 0;
-  // bf16 masks are added on the matrix core (see Attn::MMF)
-  if (p->dtype == MI355_FA_BF16 && !(p->scale_softmax < 0.99f)) return 0;
+  // bf16 masks are added on the matrix core (see Attn::MMF); the 8-wave tile
+  // kernel of 64-wide heads scales them by the fp32 1/scale where that is no bf16
+  // value, and keeps those calls
+  if (p->dtype == MI355_FA_BF16 &&
+      (!(p->scale_softmax < 0.99f) ||
+       (!forced && p->d == 64 && tile_waves == 8 && !exact_mask_weight(p->scale_softmax))))
+    return 0;
   const int64_t rows = (int64_t)(p->h / p->h_k) * p->seqlen_q, per = (rows + 31) / 32;
   const int64_t blocks = (int64_t)p->b * p->h_k * per;
   if (rows > (1 << 24) || (!forced && blocks > 16 * cus)) return 0;
@@ -2804,7 +2818,7 @@ static Plan make_plan(const mi355_fa_params* p, int cus, bool allow_stage = true
   if (pl.splits < 1) pl.splits = 1;
   const bool mask_direct = ((uintptr_t)p->mask & 15) == 0 && (p->mask_batch_stride & 7) == 0 &&
                            (p->mask_row_stride & 7) == 0;
-  pl.ks = pick_streams(p, v, cus, mask_direct, best, &pl.splits);
+  pl.ks = pick_streams(p, v, cus, mask_direct, pl.waves, best, &pl.splits);
   const int s = pl.splits;
   pl.n_per_split = (s > 1) ? ceil_div(pl.num_n, s) : pl.num_n;
   if (s > 1) {
@@ -3216,7 +3230,6 @@ static int fwd_impl(const mi355_fa_params* p, void* stream, char* err, size_t er
   kp.num_splits = pl.splits; kp.n_per_split = pl.n_per_split;
   kp.total = (int)total;
   kp.scale = p->scale_softmax;
-  kp.mask_mfma = (p->dtype == MI355_FA_BF16 && p->scale_softmax < 0.99f && !pl.mask_mfma_off) ? 1 : 0;
   kp.kv_nt = pl.kv_nt;
   {
     const float c2 = p->scale_softmax * kLog2e, slack = kRescaleSlack / p->scale_softmax;
@@ -3245,8 +3258,13 @@ static int fwd_impl(const mi355_fa_params* p, void* stream, char* err, size_t er
     kp.m_bs = (int64_t)p->seqlen_q * pl.stage_rs;
     kp.msq = p->seqlen_q;
     kp.mask_direct = 1;
-    kp.mask_clean = kp.mask_mfma;
   }
+  // bf16 masks on the matrix core weigh bf16(1/scale). 64-wide heads, 8 waves and
+  // aligned rows do so where that is 1/scale itself, else on the VALU in fp32
+  // (scale 0.09: 0.13 % of every bias).
+  kp.mask_mfma = (p->dtype == MI355_FA_BF16 && p->scale_softmax < 0.99f && !pl.mask_mfma_off &&
+                  (p->d == 128 || pl.waves == 4 || !kp.mask_direct || exact_mask_weight(p->scale_softmax))) ? 1 : 0;
+  kp.mask_clean = pl.staged && kp.mask_mfma;
 
   if (pl.scan_bytes && p->workspace && p->workspace_bytes >= pl.ws_bytes + pl.scan_bytes) {
     kp.scan_slots = (unsigned long long*)((char*)p->workspace + pl.ws_bytes);

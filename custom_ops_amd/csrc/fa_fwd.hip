@@ -166,7 +166,7 @@ struct KParams {
   const uint16_t* v;
   const uint16_t* mask;
   uint16_t* o;
-  uint16_t* o_part; // [splits][B*H][Sq][D] input dtype (split path)
+  uint16_t* o_part; // [splits][B*H][Sq][D] input dtype (split path; key streams: fp32)
   float* lse_part; // [splits][B*H][Sq]    fp32, natural log
 
   int64_t q_bs, q_hs;
@@ -2306,7 +2306,7 @@ void fa_fwd_kernel_pp(const KParams p) {
 
 // ── split-KV combine ────────────────────────────────────────────────────────
 struct CParams {
-  const uint16_t* o_part;
+  const void* o_part;    // [splits][rows][D]: 16-bit (tile kernels) or fp32 (key streams)
   const float* lse_part;
   uint16_t* o;
   int64_t o_bs, o_hs, o_rs;
@@ -2315,18 +2315,38 @@ struct CParams {
   uint32_t part_bytes;   // bytes of o_part when below 2^31 (buffer-addressed loads), else 0
 };
 
-// Workgroup = kCombineThreads / (D/8) rows × D columns: 256 threads (16 rows
-// at d = 128) for large grids, one wave (4 rows) when that would leave fewer
+// 16 bytes of a partial row: 8 values in the element type (tile kernels, as the
+// reference stores them), or 4 in fp32 (P32, key streams: they split calls that
+// the tile plan runs unsplit, with O in fp32 throughout; 16-bit partials made
+// [19,12/4,1,1808,64]'s error 1.2 times the unsplit one)
+template <bool BF16, bool P32> struct Part {
+  static constexpr int kV = P32 ? 4 : 8;
+  static constexpr uint32_t kBytes = P32 ? 4 : 2;   // per value
+  typedef float F __attribute__((ext_vector_type(kV)));
+  typedef typename std::conditional<BF16, __bf16, _Float16>::type E;
+  typedef E EV __attribute__((ext_vector_type(kV)));
+  static __device__ __forceinline__ F get(u32x4 raw) {
+    if constexpr (P32) return bitcast<F>(raw);
+    else return __builtin_convertvector(bitcast<EV>(raw), F);
+  }
+  static __device__ __forceinline__ void store(uint16_t* dst, F x) {
+    *reinterpret_cast<EV*>(dst) = __builtin_convertvector(x, EV);
+  }
+};
+
+// Workgroup = kCombineThreads / (D/8) rows × D columns (fp32 partials: D/4): 256
+// threads (16 rows at d = 128) for large grids, one wave (4 rows) when that would leave fewer
 // than 1024 workgroups, so a small split grid still fills the chip; thread = 8
-// consecutive d-values of a row (one 16-byte load per split). Phase 1 stages the rows' LSEs in LDS and turns
+// (fp32: 4) consecutive d-values of a row (one 16-byte load per split). Phase 1 stages the rows' LSEs in LDS and turns
 // them into weights w_s = exp(lse_s − max) / Σ (all-(-inf) row → all weights
 // 0 → output 0); phase 2 accumulates Σ w_s·O_s in fp32 with up to 16 (one
 // wave) or 8 (256 threads) splits' loads in flight (more spills SGPRs). (Issuing them before phase 1 is slower: loads complete in
 // order, so the LSE reads would wait behind them.)
-template <int D, bool BF16, int kCombineThreads>
+template <int D, bool BF16, bool P32, int kCombineThreads>
 __global__ __launch_bounds__(kCombineThreads) void fa_combine_kernel(const CParams p) {
-  typedef typename Elt<BF16>::v8 V8;
-  constexpr int kTPR = D / 8;                     // threads per row
+  typedef Part<BF16, P32> Pt;
+  typedef typename Pt::F F;
+  constexpr int kTPR = D / Pt::kV;                     // threads per row
   constexpr int kRows = kCombineThreads / kTPR;   // rows per workgroup
   // splits' loads in flight per thread: all of a typical small grid's splits
   // in one round trip for the one-wave variant; 8 keeps the large-grid
@@ -2346,12 +2366,12 @@ __global__ __launch_bounds__(kCombineThreads) void fa_combine_kernel(const CPara
     // arithmetic in the same order (bit-identical). cfg5 (2 splits, combine
     // launch after the ping-pong loop): 44.5 -> 43.1 µs hot; cfg4 (16
     // splits, one-wave workgroups): 1-2 µs faster.
-    const int r = tid / kTPR, c8 = tid % kTPR;
+    const int r = tid / kTPR, cv = tid % kTPR;
     const int64_t row = row0 + r;
     if (row >= p.rows) return;
     const rsrc_t rp = make_rsrc(p.o_part, p.part_bytes);
-    const uint32_t off0 = (uint32_t)((row * D + c8 * 8) * 2);
-    const uint32_t sstep = (uint32_t)(slab * D * 2);
+    const uint32_t off0 = (uint32_t)(row * D + cv * Pt::kV) * Pt::kBytes;
+    const uint32_t sstep = (uint32_t)(slab * D) * Pt::kBytes;
     float l[kOnePass];
     u32x4 raw[kOnePass];
 #pragma unroll
@@ -2370,14 +2390,14 @@ __global__ __launch_bounds__(kCombineThreads) void fa_combine_kernel(const CPara
       sum += w[u];
     }
     const float inv = (sum > 0.f) ? 1.f / sum : 0.f;
-    f32x8 acc = {};
+    F acc = {};
 #pragma unroll
-    for (int u = 0; u < kOnePass; ++u) acc += (w[u] * inv) * __builtin_convertvector(bitcast<V8>(raw[u]), f32x8);
+    for (int u = 0; u < kOnePass; ++u) acc += (w[u] * inv) * Pt::get(raw[u]);
     const int64_t bh = row / p.sq;
     const int m = (int)(row % p.sq);
     const int b = (int)(bh / p.h), h = (int)(bh % p.h);
-    uint16_t* dst = p.o + (int64_t)b * p.o_bs + (int64_t)h * p.o_hs + (int64_t)m * p.o_rs + c8 * 8;
-    *reinterpret_cast<u32x4*>(dst) = bitcast<u32x4>(__builtin_convertvector(acc, V8));
+    uint16_t* dst = p.o + (int64_t)b * p.o_bs + (int64_t)h * p.o_hs + (int64_t)m * p.o_rs + cv * Pt::kV;
+    Pt::store(dst, acc);
     return;
   }
   for (int i = tid; i < S * kRows; i += kCombineThreads) {
@@ -2401,11 +2421,11 @@ __global__ __launch_bounds__(kCombineThreads) void fa_combine_kernel(const CPara
   }
   __syncthreads();
   const int r = tid / kTPR;
-  const int c8 = tid % kTPR;
+  const int cv = tid % kTPR;
   const int64_t row = row0 + r;
   if (row >= p.rows) return;
-  const uint16_t* src = p.o_part + row * D + c8 * 8;
-  f32x8 acc = {};
+  const char* src = static_cast<const char*>(p.o_part) + (row * D + cv * Pt::kV) * Pt::kBytes;
+  F acc = {};
   // A split with weight 0 (lse = -inf: no live key of the row in that split,
   // e.g. outside a sliding window) adds exactly nothing, so its partial is not
   // fetched (cf. the active-split mask of csrc/fa/sm89/fa_fwd_kernel.h:1458-1468;
@@ -2414,8 +2434,8 @@ __global__ __launch_bounds__(kCombineThreads) void fa_combine_kernel(const CPara
   // memory access, keeping every split's load of the batch in flight together.
   if (p.part_bytes) {
     const rsrc_t rp = make_rsrc(p.o_part, p.part_bytes);
-    const uint32_t off0 = (uint32_t)((row * D + c8 * 8) * 2);
-    const uint32_t sstep = (uint32_t)(slab * D * 2);
+    const uint32_t off0 = (uint32_t)(row * D + cv * Pt::kV) * Pt::kBytes;
+    const uint32_t sstep = (uint32_t)(slab * D) * Pt::kBytes;
     for (int s0 = 0; s0 < S; s0 += kBatch) {
       u32x4 raw[kBatch];
       float w[kBatch];
@@ -2425,41 +2445,42 @@ __global__ __launch_bounds__(kCombineThreads) void fa_combine_kernel(const CPara
         raw[u] = bload16(rp, w[u] != 0.f ? off0 + (uint32_t)(s0 + u) * sstep : 0x80000000u);
       }
 #pragma unroll
-      for (int u = 0; u < kBatch; ++u) acc += w[u] * __builtin_convertvector(bitcast<V8>(raw[u]), f32x8);
+      for (int u = 0; u < kBatch; ++u) acc += w[u] * Pt::get(raw[u]);
     }
   } else {
     for (int s0 = 0; s0 < S; s0 += kBatch) {
       u32x4 raw[kBatch];
 #pragma unroll
       for (int u = 0; u < kBatch; ++u)
-        if (s0 + u < S) raw[u] = *reinterpret_cast<const u32x4*>(src + (int64_t)(s0 + u) * slab * D);
+        if (s0 + u < S) raw[u] = *reinterpret_cast<const u32x4*>(src + (int64_t)(s0 + u) * slab * D * Pt::kBytes);
 #pragma unroll
       for (int u = 0; u < kBatch; ++u)
-        if (s0 + u < S) acc += sw[(s0 + u) * kRows + r] * __builtin_convertvector(bitcast<V8>(raw[u]), f32x8);
+        if (s0 + u < S) acc += sw[(s0 + u) * kRows + r] * Pt::get(raw[u]);
     }
   }
   const int64_t bh = row / p.sq;
   const int m = (int)(row % p.sq);
   const int b = (int)(bh / p.h), h = (int)(bh % p.h);
-  uint16_t* dst = p.o + (int64_t)b * p.o_bs + (int64_t)h * p.o_hs + (int64_t)m * p.o_rs + c8 * 8;
-  *reinterpret_cast<u32x4*>(dst) = bitcast<u32x4>(__builtin_convertvector(acc, V8));
+  uint16_t* dst = p.o + (int64_t)b * p.o_bs + (int64_t)h * p.o_hs + (int64_t)m * p.o_rs + cv * Pt::kV;
+  Pt::store(dst, acc);
 }
 
 // More than 16 splits on a small grid (one-wave workgroups): four waves per
-// 64 / (D / 8) rows, each with up to 16 splits' LSEs and partial slices in one
+// 64 / (D / 8) rows (fp32 partials: D / 4), each with up to 16 splits' LSEs and partial slices in one
 // round trip and its own running max; the four sums then meet in LDS.
-template <int D, bool BF16>
+template <int D, bool BF16, bool P32>
 __global__ __launch_bounds__(256) void fa_combine_wide_kernel(const CParams p) {
-  typedef typename Elt<BF16>::v8 V8;
-  constexpr int kTPR = D / 8, kRows = 64 / kTPR, kPer = kMaxSplits / 4;
-  __shared__ __align__(16) f32x8 sacc[4][64];
+  typedef Part<BF16, P32> Pt;
+  typedef typename Pt::F F;
+  constexpr int kTPR = D / Pt::kV, kRows = 64 / kTPR, kPer = kMaxSplits / 4;
+  __shared__ __align__(16) F sacc[4][64];
   __shared__ float sml[4][2][kRows];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int r = lane / kTPR, c8 = lane % kTPR;
+  const int r = lane / kTPR, cv = lane % kTPR;
   const int64_t row = (int64_t)blockIdx.x * kRows + r;
   const bool in = row < p.rows;
   const int per = (p.num_splits + 3) / 4, s0 = wave * per, s1 = min(s0 + per, p.num_splits);
-  const uint32_t sstep = (uint32_t)(p.rows * D * 2), off0 = (uint32_t)((row * D + c8 * 8) * 2);
+  const uint32_t sstep = (uint32_t)(p.rows * D) * Pt::kBytes, off0 = (uint32_t)(row * D + cv * Pt::kV) * Pt::kBytes;
   const rsrc_t rp = make_rsrc(p.o_part, p.part_bytes);
   float l[kPer];
   u32x4 raw[kPer];
@@ -2473,23 +2494,23 @@ __global__ __launch_bounds__(256) void fa_combine_wide_kernel(const CParams p) {
 #pragma unroll
   for (int u = 0; u < kPer; ++u) mx = fmaxf(mx, l[u]);
   const float mxc = (mx == -INFINITY) ? 0.f : mx;
-  f32x8 acc = {};
+  F acc = {};
   float sum = 0.f;
 #pragma unroll
   for (int u = 0; u < kPer; ++u) {
     const float w = __builtin_amdgcn_exp2f((l[u] - mxc) * kLog2e);
     sum += w;
-    acc += w * __builtin_convertvector(bitcast<V8>(raw[u]), f32x8);
+    acc += w * Pt::get(raw[u]);
   }
   sacc[wave][lane] = acc;
-  if (c8 == 0) { sml[wave][0][r] = mx; sml[wave][1][r] = sum; }
+  if (cv == 0) { sml[wave][0][r] = mx; sml[wave][1][r] = sum; }
   __syncthreads();
   if (wave != 0 || !in) return;
   float m4 = -INFINITY;
 #pragma unroll
   for (int w = 0; w < 4; ++w) m4 = fmaxf(m4, sml[w][0][r]);
   const float m4c = (m4 == -INFINITY) ? 0.f : m4;
-  f32x8 o = {};
+  F o = {};
   float total = 0.f;
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
@@ -2500,8 +2521,8 @@ __global__ __launch_bounds__(256) void fa_combine_wide_kernel(const CParams p) {
   o *= (total > 0.f) ? 1.f / total : 0.f;
   const int64_t bh = row / p.sq;
   const int m = (int)(row % p.sq), b = (int)(bh / p.h), h = (int)(bh % p.h);
-  uint16_t* dst = p.o + (int64_t)b * p.o_bs + (int64_t)h * p.o_hs + (int64_t)m * p.o_rs + c8 * 8;
-  *reinterpret_cast<u32x4*>(dst) = bitcast<u32x4>(__builtin_convertvector(o, V8));
+  uint16_t* dst = p.o + (int64_t)b * p.o_bs + (int64_t)h * p.o_hs + (int64_t)m * p.o_rs + cv * Pt::kV;
+  Pt::store(dst, o);
 }
 
 // ════════════════════════════════════════════════════════════════════════════
@@ -2823,7 +2844,7 @@ static Plan make_plan(const mi355_fa_params* p, int cus, bool allow_stage = true
   pl.n_per_split = (s > 1) ? ceil_div(pl.num_n, s) : pl.num_n;
   if (s > 1) {
     const size_t rows = (size_t)s * p->b * p->h * p->seqlen_q;
-    pl.o_part_bytes = (rows * p->d * sizeof(uint16_t) + 255) & ~(size_t)255;
+    pl.o_part_bytes = (rows * p->d * (pl.ks ? sizeof(float) : sizeof(uint16_t)) + 255) & ~(size_t)255;
     pl.lse_bytes = (rows * sizeof(float) + 255) & ~(size_t)255;
   }
   if (pl.ks) {   // 32 flattened rows per workgroup; the mask is read in place, no live ranges
@@ -3079,18 +3100,18 @@ static hipError_t launch_variant(const KParams& kp, const Plan& pl, hipStream_t 
   return pl.deep ? launch_main<D, BF16, SPLIT, 4, true>(kp, st) : launch_main<D, BF16, SPLIT, 4, false>(kp, st);
 }
 
-template <int D, bool BF16>
+template <int D, bool BF16, bool P32>
 static hipError_t launch_combine(const CParams& cp, hipStream_t st) {
   // 256-thread workgroups while they still number >= 1024, else one wave each.
-  constexpr int kRows256 = 256 / (D / 8), kRows64 = 64 / (D / 8);
+  constexpr int kTPR = D / Part<BF16, P32>::kV, kRows256 = 256 / kTPR, kRows64 = 64 / kTPR;
   if ((cp.rows + kRows256 - 1) / kRows256 >= 1024) {
-    hipLaunchKernelGGL((fa_combine_kernel<D, BF16, 256>),
+    hipLaunchKernelGGL((fa_combine_kernel<D, BF16, P32, 256>),
                        dim3((unsigned)((cp.rows + kRows256 - 1) / kRows256)), dim3(256), 0, st, cp);
   } else if (cp.num_splits > 16 && cp.part_bytes) {
-    hipLaunchKernelGGL((fa_combine_wide_kernel<D, BF16>),
+    hipLaunchKernelGGL((fa_combine_wide_kernel<D, BF16, P32>),
                        dim3((unsigned)((cp.rows + kRows64 - 1) / kRows64)), dim3(256), 0, st, cp);
   } else {
-    hipLaunchKernelGGL((fa_combine_kernel<D, BF16, 64>),
+    hipLaunchKernelGGL((fa_combine_kernel<D, BF16, P32, 64>),
                        dim3((unsigned)((cp.rows + kRows64 - 1) / kRows64)), dim3(64), 0, st, cp);
   }
   return hipGetLastError();
@@ -3113,7 +3134,7 @@ static hipError_t launch(const KParams& kp_in, const CParams& cp, const Plan& pl
     if (kp.mask_direct) launch_streams<D, BF16, true>(kp, pl.ks, st);
     else launch_streams<D, BF16, false>(kp, pl.ks, st);
     const hipError_t e = hipGetLastError();
-    return e != hipSuccess || !split ? e : launch_combine<D, BF16>(cp, st);
+    return e != hipSuccess || !split ? e : launch_combine<D, BF16, true>(cp, st);
   }
   const int lm = pl.live;
   const bool pp = D == 128 && BF16 && pl.loop == 3 && runs_asm_loop<D, BF16>(kp, pl);
@@ -3138,7 +3159,7 @@ static hipError_t launch(const KParams& kp_in, const CParams& cp, const Plan& pl
   kf.fuse = kp.fuse && !runs_asm_loop<D, BF16>(kp, pl);
   hipError_t e = launch_variant<D, BF16, true>(kf, pl, st);
   if (e != hipSuccess || kf.fuse) return e;
-  return launch_combine<D, BF16>(cp, st);
+  return launch_combine<D, BF16, false>(cp, st);
 }
 
 }  // namespace mi355fa

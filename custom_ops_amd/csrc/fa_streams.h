@@ -284,43 +284,53 @@ __device__ __forceinline__ void stream_merge(const StreamRows<D, BF16>& a, uint8
     l = __builtin_fmaf(mw[w], sml[(w * RG + rg) * 64 + 32 + l32], l);
   }
   const float inv = (l == 0.f || l != l) ? 1.f : 1.f / l;
-  u32x2 out[kPer];
+  f32x4 out[kPer];
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
     f32x4 acc = {};
 #pragma unroll
     for (int w = 0; w < KG; ++w)
       acc += mw[w] * *reinterpret_cast<const f32x4*>(smem + (((w * RG + rg) * kQuads + kg * kPer + j) * 64 + lane) * 16);
-    acc *= inv;
-    typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-    typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
-    if constexpr (BF16) out[j] = bitcast<u32x2>(__builtin_convertvector(acc, bf16x4));
-    else out[j] = bitcast<u32x2>(__builtin_convertvector(acc, f16x4));
+    out[j] = acc * inv;
   }
   const kernarg_ptr p = reload_params();
   const StreamIdx ix = StreamIdx::of<RG>(p);
   int h, m;
   const int r = ix.row0 + rg * 32 + l32;
   ix.row(r, h, m);
-  const bool in = r < ix.rows, split = p->num_splits > 1;
-  const int64_t prow = (((int64_t)ix.split * p->b + ix.b) * p->h + h) * p->sq + m;
-  uint16_t* dst = split ? p->o_part + prow * D
-                        : p->o + (int64_t)ix.b * p->o_bs + (int64_t)h * p->o_hs + (int64_t)m * p->o_rs;
-  // quad j holds d = 8j + 4g .. +3 of the lane's row; two quads exchanged with
-  // the lane 32 apart make a 16-byte chunk per lane (chunk j below, j + 1 above)
+  const bool in = r < ix.rows;
+  // quad j holds d = 8j + 4g .. +3 of the lane's row
+  if (p->num_splits > 1) {   // the split's partial: fp32, with its LSE
+    const int64_t prow = (((int64_t)ix.split * p->b + ix.b) * p->h + h) * p->sq + m;
+    float* dst = reinterpret_cast<float*>(p->o_part) + prow * D + kg * kPer * 8 + g * 4;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j)
+      if (in) *reinterpret_cast<f32x4*>(dst + j * 8) = out[j];
+    if (kg == 0 && g == 0 && in)
+      p->lse_part[prow] = (l == 0.f || l != l) ? -INFINITY
+                         : __builtin_fmaf(mx, p->scale, __builtin_amdgcn_logf(l) * 0.69314718f);
+    return;
+  }
+  typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+  typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
+  auto half = [&](int j) {
+    if constexpr (BF16) return bitcast<u32x2>(__builtin_convertvector(out[j], bf16x4));
+    else return bitcast<u32x2>(__builtin_convertvector(out[j], f16x4));
+  };
+  uint16_t* dst = p->o + (int64_t)ix.b * p->o_bs + (int64_t)h * p->o_hs + (int64_t)m * p->o_rs;
+  // two quads exchanged with the lane 32 apart make a 16-byte chunk per lane
+  // (chunk j below, j + 1 above)
   if constexpr (kPer >= 2) {
 #pragma unroll
     for (int j = 0; j < kPer; j += 2) {
-      const auto s0 = __builtin_amdgcn_permlane32_swap(out[j][0], out[j + 1][0], false, false);
-      const auto s1 = __builtin_amdgcn_permlane32_swap(out[j][1], out[j + 1][1], false, false);
+      const u32x2 lo = half(j), hi = half(j + 1);
+      const auto s0 = __builtin_amdgcn_permlane32_swap(lo[0], hi[0], false, false);
+      const auto s1 = __builtin_amdgcn_permlane32_swap(lo[1], hi[1], false, false);
       if (in) *reinterpret_cast<u32x4*>(dst + (kg * kPer + j + g) * 8) = u32x4{s0[0], s1[0], s0[1], s1[1]};
     }
   } else {
-    if (in) *reinterpret_cast<u32x2*>(dst + kg * 8 + g * 4) = out[0];
+    if (in) *reinterpret_cast<u32x2*>(dst + kg * 8 + g * 4) = half(0);
   }
-  if (split && kg == 0 && g == 0 && in)
-    p->lse_part[prow] = (l == 0.f || l != l) ? -INFINITY
-                       : __builtin_fmaf(mx, p->scale, __builtin_amdgcn_logf(l) * 0.69314718f);
 }
 
 // RG = 1: every wave is a key group of its own, with its own waits and no

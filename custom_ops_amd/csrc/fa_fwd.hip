@@ -3371,8 +3371,10 @@ extern "C" int mi355_fa_fwd_noalloc(const mi355_fa_params* p, void* stream, char
   int rc = validate(p, err, errlen);
   if (rc) return rc;
   if (p->b == 0 || p->h == 0 || p->seqlen_q == 0) return MI355_FA_OK;
-  // the staged mask when it fits the scratch, else the mask read in place
-  size_t need = mi355_fa_workspace_bytes(p);
+  // the staged mask when it fits the scratch, else the mask read in place. What
+  // a launch can do without (the shared scan's words) stays out of the array: a
+  // call that needs nothing from it cannot race with one that does.
+  size_t need = plan_for(p, device_info().cus).ws_bytes;
   bool allow_stage = true;
   if (need > MI355_FA_NOALLOC_SCRATCH_BYTES) {
     allow_stage = false;
@@ -3391,7 +3393,7 @@ extern "C" int mi355_fa_fwd_noalloc(const mi355_fa_params* p, void* stream, char
   if (need > 0) {
     rc = scratch_of_current_device(&q.workspace, err, errlen);
     if (rc) return rc;
-    q.workspace_bytes = MI355_FA_NOALLOC_SCRATCH_BYTES;
+    q.workspace_bytes = need;
   }
   return fwd_impl(&q, stream, err, errlen, allow_stage);
 }

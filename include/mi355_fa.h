@@ -131,9 +131,11 @@ int mi355_fa_fwd(const mi355_fa_params* p, void* stream, char* err, size_t errle
  * device array of MI355_FA_NOALLOC_SCRATCH_BYTES (allocated when the
  * library's code is loaded onto a GPU and held until the process ends).
  * p->workspace is ignored. A staged mask that does not fit is read in place
- * instead; plans that still need more scratch fail with MI355_FA_EWORKSPACE. Calls that overlap on
- * one GPU (other streams, other threads) share the array and race: serialise
- * them. No counterpart in the reference; it is for callers that cannot
+ * instead; plans that still need more scratch fail with MI355_FA_EWORKSPACE.
+ * The optional words of large unsplit launches (mi355_fa_workspace_bytes) are
+ * done without, so calls that need no workspace leave the array alone. Calls
+ * that do and overlap on one GPU (other streams, other threads) share the
+ * array and race: serialise them. No counterpart in the reference; it is for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc). */
 int mi355_fa_fwd_noalloc(const mi355_fa_params* p, void* stream, char* err, size_t errlen);

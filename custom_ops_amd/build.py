@@ -9,7 +9,9 @@ violates those properties.
 from __future__ import annotations
 
 import glob
+import hashlib
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -88,30 +90,69 @@ TORCH_BINDING_PATH = os.path.join(PKG_DIR, "libmi355_fa_torch.so")
 OPS_PATH = os.path.join(PKG_DIR, "libmi355_fa_ops.so")   # the same source, implementation only
 
 
-def build_torch_binding(verbose: bool = False) -> str:
-    """Compile the C++ torch extension over the C ABI (csrc/torch_binding.cpp:
-    the reference-style TORCH_LIBRARY binding) against this PyTorch-ROCm, linked
-    to libmi355_fa.so next to it, and the implementation-only form that fa.py
-    binds to the library it opened. Host code only, so the host compiler builds it."""
+def ops_stamp() -> str:
+    """What a compiled operator implementation has to be built from: its sources
+    and the PyTorch it runs in. The file holds this text (csrc/torch_binding.cpp)."""
+    import torch
+    h = hashlib.sha256()
+    for src in (TORCH_BINDING_SRC, os.path.join(INCLUDE, "mi355_fa.h")):
+        with open(src, "rb") as f:
+            h.update(f.read())
+    return f"mi355-ops {h.hexdigest()} torch {torch.__version__};"
+
+
+def ops_stamp_of(path: str) -> str | None:
+    """The stamp in a built file, read without opening it as a library; None
+    where the file is missing or holds none."""
+    try:
+        with open(path, "rb") as f:
+            found = re.search(rb"mi355-ops [0-9a-f]{64} torch [^;\0]{1,64};", f.read())
+    except OSError:
+        return None
+    return found.group().decode(errors="replace") if found else None
+
+
+def ops_current(path: str) -> bool:
+    """Whether the file was built from the present sources for this PyTorch."""
+    try:
+        return ops_stamp_of(path) == ops_stamp()
+    except OSError:      # no sources to compare with
+        return False
+
+
+def _compile_binding(path: str, extra: list, verbose: bool) -> str:
     import torch
     tdir = os.path.dirname(torch.__file__)
     abi = int(torch.compiled_with_cxx11_abi())
     cxx = os.environ.get("CXX") or shutil.which("g++") or "g++"
-    common = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
-              f"-D_GLIBCXX_USE_CXX11_ABI={abi}", f"-I{tdir}/include",
-              f"-I{tdir}/include/torch/csrc/api/include", "-I/opt/rocm/include", f"-I{INCLUDE}",
-              TORCH_BINDING_SRC]
-    libs = [f"-L{tdir}/lib", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip",
-            "-L/opt/rocm/lib", "-lamdhip64"]
-    for path, extra in ((TORCH_BINDING_PATH, [f"-L{PKG_DIR}", "-lmi355_fa", "-Wl,-rpath,$ORIGIN"]),
-                        (OPS_PATH, ["-DMI355_OPS_IMPL_ONLY"])):
-        cmd = [*common, "-o", path + ".tmp", *libs, *extra]
-        if verbose:
-            print(" ".join(cmd), flush=True)
-        res = subprocess.run(cmd, capture_output=True, text=True)
-        if res.returncode != 0:
-            raise RuntimeError(f"torch binding build failed ({res.returncode}):\n{res.stderr[-4000:]}")
-        os.replace(path + ".tmp", path)
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+           f"-D_GLIBCXX_USE_CXX11_ABI={abi}", f"-I{tdir}/include",
+           f"-I{tdir}/include/torch/csrc/api/include", "-I/opt/rocm/include", f"-I{INCLUDE}",
+           TORCH_BINDING_SRC, "-o", path + ".tmp",
+           f"-L{tdir}/lib", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip",
+           "-L/opt/rocm/lib", "-lamdhip64", *extra]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"torch binding build failed ({res.returncode}):\n{res.stderr[-4000:]}")
+    os.replace(path + ".tmp", path)
+    return path
+
+
+def build_ops(path: str = OPS_PATH, verbose: bool = False) -> str:
+    """Compile the operator's implementation alone, which the loader binds to the
+    library it opened."""
+    return _compile_binding(path, ["-DMI355_OPS_IMPL_ONLY", f'-DMI355_OPS_STAMP="{ops_stamp()}"'], verbose)
+
+
+def build_torch_binding(verbose: bool = False) -> str:
+    """Compile the C++ torch extension over the C ABI (csrc/torch_binding.cpp:
+    the reference-style TORCH_LIBRARY binding) against this PyTorch-ROCm, linked
+    to libmi355_fa.so next to it, and the implementation-only form. Host code
+    only, so the host compiler builds both."""
+    _compile_binding(TORCH_BINDING_PATH, [f"-L{PKG_DIR}", "-lmi355_fa", "-Wl,-rpath,$ORIGIN"], verbose)
+    build_ops(verbose=verbose)
     return TORCH_BINDING_PATH
 
 

@@ -10,8 +10,10 @@
 //
 // Compiled a second time with MI355_OPS_IMPL_ONLY (libmi355_fa_ops.so), the same
 // function is only the CUDA-key implementation of the operator that fa.py has
-// defined, and reaches the library that fa.py opened through two addresses
-// (mi355_ops_bind). A call of a small problem costs its host work: through the
+// defined, and reaches the library that fa.py opened through two addresses.
+// mi355_ops_connect registers it, so that opening the file changes nothing in the
+// dispatcher; the file names the sources and the PyTorch it was built from
+// (mi355_ops_stamp), which are read before it is opened. A call of a small problem costs its host work: through the
 // Python implementation and ctypes [1,8,100,200] took 12.5 µs a call, its
 // kernel 7.5.
 //
@@ -114,14 +116,27 @@ at::Tensor mha_fwd_with_mask_mi355(const at::Tensor& q, const at::Tensor& k,
 }  // namespace
 
 #ifdef MI355_OPS_IMPL_ONLY
-// The opened library's entry points, set once before the operator is called.
-extern "C" void mi355_ops_bind(void* fwd, void* workspace_bytes) {
+extern "C" __attribute__((used, visibility("default"))) const char mi355_ops_stamp[] = MI355_OPS_STAMP;
+
+// Takes the opened library's entry points and registers the implementation, once.
+// abi and params_bytes are the caller's: 1 (and nothing registered) where this
+// file was compiled for another ABI version or parameter layout.
+extern "C" int mi355_ops_connect(void* fwd, void* workspace_bytes, int abi, size_t params_bytes) {
+  if (abi != MI355_FA_ABI_VERSION || params_bytes != sizeof(mi355_fa_params)) return 1;
   g_fwd = reinterpret_cast<decltype(g_fwd)>(fwd);
   g_workspace_bytes = reinterpret_cast<decltype(g_workspace_bytes)>(workspace_bytes);
+  try {
+    static torch::Library lib(torch::Library::IMPL, "recsys_ops", c10::DispatchKey::CUDA, __FILE__, __LINE__);
+    static const bool once = (lib.impl("mha_fwd_with_mask", &mha_fwd_with_mask_mi355), true);
+    (void)once;
+  } catch (const std::exception&) {
+    return 1;
+  }
+  return 0;
 }
 #else
 TORCH_LIBRARY_FRAGMENT(recsys_ops, m) {
   m.def("mha_fwd_with_mask(Tensor q, Tensor k, Tensor v, Tensor mask) -> Tensor");
 }
-#endif
 TORCH_LIBRARY_IMPL(recsys_ops, CUDA, m) { m.impl("mha_fwd_with_mask", &mha_fwd_with_mask_mi355); }
+#endif

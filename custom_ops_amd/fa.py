@@ -22,7 +22,6 @@ from __future__ import annotations
 
 import ctypes
 import math
-import os
 
 import torch
 
@@ -173,26 +172,31 @@ def _cuda_impl(q, k, v, mask):
 _registered = False
 _torch_lib = None
 _ops_lib = None
+native_path = None   # the compiled implementation to open, set by the loader once it is checked
 
 
 def _bind_native() -> bool:
-    """Load the compiled CUDA-key implementation (csrc/torch_binding.cpp built
-    implementation-only: the checks, workspace and launch of
-    ``mha_fwd_with_mask_hip`` in C++) and hand it the opened library's entry
-    points. False where it was not built against this PyTorch: the Python
-    implementation, which calls the same library, then serves."""
+    """Open the compiled CUDA-key implementation that the loader named
+    (``native_path``: csrc/torch_binding.cpp built implementation-only, the
+    checks, workspace and launch of ``mha_fwd_with_mask_hip`` in C++) and hand
+    it the opened library's entry points. False where there is none for this
+    process, or for another ABI: the Python implementation, which calls the same
+    library, then serves."""
     global _ops_lib
-    if not os.path.exists(OPS_PATH):
+    if native_path is None:
         return False
     lib = _lib.load()
     try:
-        ops = ctypes.CDLL(OPS_PATH)
-    except OSError:
+        ops = ctypes.CDLL(native_path)
+        connect = ops.mi355_ops_connect
+    except (OSError, AttributeError):
         return False
-    ops.mi355_ops_bind.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
-    ops.mi355_ops_bind.restype = None
-    ops.mi355_ops_bind(ctypes.cast(lib.mi355_fa_fwd, ctypes.c_void_p),
-                       ctypes.cast(lib.mi355_fa_workspace_bytes, ctypes.c_void_p))
+    connect.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t]
+    connect.restype = ctypes.c_int
+    if connect(ctypes.cast(lib.mi355_fa_fwd, ctypes.c_void_p),
+               ctypes.cast(lib.mi355_fa_workspace_bytes, ctypes.c_void_p),
+               _lib.ABI_VERSION, ctypes.sizeof(_lib.Params)) != 0:
+        return False
     _ops_lib = ops
     return True
 

@@ -16,9 +16,11 @@ This module's own design for that contract:
   sections — ``contract`` (operator namespace, schemas, Meta ops, C ABI),
   ``runtime`` (torch major.minor, HIP major), ``targets`` (gfx names) and
   ``provenance`` (sources digest, flags, compiler) — plus ``payload`` (file
-  name, size, SHA-256). ``seal`` is the SHA-256 of the canonical JSON of all
-  of them, so any edit of the sidecar is caught before its content is
-  trusted.
+  name, size, SHA-256) and, where the build made one, ``companion`` (the same
+  for the compiled operator implementation next to the library). ``seal`` is
+  the SHA-256 of the canonical JSON of all of them, so any edit of the sidecar
+  is caught before its content is trusted. A compiled implementation that no
+  sealed section names is never opened in strict mode.
 * Validation is a table of named checks (``_CHECKS``), each comparing one
   section with what this process expects and returning a message, so the
   error says which section disagreed and how.
@@ -173,6 +175,26 @@ def _check_payload(md: dict, exp: _Expectation, lib: Path) -> Optional[str]:
     return None
 
 
+def _companion(md: dict, lib: Path) -> Optional[Path]:
+    """The compiled operator implementation that was deployed with ``lib`` (None:
+    not built, not deployed, or built for another PyTorch)."""
+    c = md.get("companion")
+    if not isinstance(c, dict) or c.get("torch") != torch.__version__ or not isinstance(c.get("file"), str):
+        return None
+    path = lib.parent / Path(c["file"]).name
+    return path if path.is_file() else None
+
+
+def _check_companion(md: dict, exp: _Expectation, lib: Path) -> Optional[str]:
+    path = _companion(md, lib)
+    if path is None:
+        return None
+    c = md["companion"]
+    if c.get("bytes") != path.stat().st_size or c.get("sha256") != _digest_file(path):
+        return f"companion digest mismatch: {path.name} differs from the one built"
+    return None
+
+
 _CHECKS: tuple = (
     ("format", _check_format),
     ("seal", _check_seal),
@@ -180,6 +202,7 @@ _CHECKS: tuple = (
     ("runtime", _check_runtime),
     ("targets", _check_targets),
     ("payload", _check_payload),
+    ("companion", _check_companion),
 )
 
 
@@ -321,9 +344,11 @@ class FAOps:
 
     def build(self, output_directory, *, offload_arch: Optional[str] = None,
               extra_flags=(), verbose: bool = False) -> Path:
-        """Compile ``<so_name>.so`` for the targets and publish its sealed sidecar
-        ``<so_name>.so.json`` next to it, without loading it. hipcc
-        cross-compiles, so no GPU is needed. Deploy both files together."""
+        """Compile ``<so_name>.so`` for the targets and the operator implementation
+        over it (``<so_name>_ops.so``, optional in a deployment: without it the
+        Python implementation serves), and publish the sealed sidecar
+        ``<so_name>.so.json`` next to them, without loading anything. hipcc
+        cross-compiles, so no GPU is needed. Deploy the files together."""
         targets = _targets(offload_arch or list(self.default_targets))
         if not targets:
             raise CustomOpsError("no offload target given")
@@ -360,9 +385,19 @@ class FAOps:
                                 "payload": {"file": library.name,
                                             "bytes": product.stat().st_size,
                                             "sha256": _digest_file(product)}}
+                    ops = out / f"{self.so_name}_ops.so"
+                    ops_product = Path(tmp) / ops.name
+                    try:
+                        _build.build_ops(str(ops_product), verbose=verbose)
+                    except RuntimeError as e:
+                        raise CustomOpsError(str(e)) from e
+                    manifest["companion"] = {"file": ops.name, "bytes": ops_product.stat().st_size,
+                                             "sha256": _digest_file(ops_product),
+                                             "torch": torch.__version__}
                     manifest["seal"] = seal_of(manifest)
                     staged = Path(tmp) / "sidecar.json"
                     staged.write_text(json.dumps(manifest, sort_keys=True, indent=2) + "\n")
+                    os.replace(ops_product, ops)
                     os.replace(product, library)
                     os.replace(staged, sidecar)
             finally:
@@ -370,7 +405,8 @@ class FAOps:
         return library
 
     # loading
-    def _validate(self, library: Path, sidecar: Path) -> None:
+    def _validate(self, library: Path, sidecar: Path) -> Optional[Path]:
+        """Run every check; returns the compiled operator implementation to open, if any."""
         try:
             md = json.loads(sidecar.read_text())
         except (OSError, ValueError) as e:
@@ -382,6 +418,7 @@ class FAOps:
             msg = check(md, exp, library)
             if msg:
                 raise CustomOpsError(f"{name} check: {msg}")
+        return _companion(md, library)
 
     def _verify_registered(self) -> None:
         for qualified, schema in self.contract()["schemas"].items():
@@ -392,8 +429,9 @@ class FAOps:
             if not torch._C._dispatch_has_kernel_for_dispatch_key(f"{self.namespace}::{op}", "Meta"):
                 raise CustomOpsError(f"no Meta (fake) kernel for {self.namespace}::{op}")
 
-    def _bind(self, library: Path, prevalidated: Callable[[], None]) -> None:
-        """Claim the operators, open the library, register and verify, in that order."""
+    def _bind(self, library: Path, native: Optional[Path], prevalidated: Callable[[], None]) -> None:
+        """Claim the operators, open the library, register (with the compiled
+        implementation at ``native``, if any) and verify, in that order."""
         prevalidated()
         identity = _identity(library)
         claims = _claim(self._qualified(), library, identity)
@@ -401,6 +439,7 @@ class FAOps:
             return
         try:
             _lib.load(str(library))
+            fa.native_path = None if native is None else str(native)
             fa.register()
             self._verify_registered()
         except Exception as e:
@@ -423,15 +462,18 @@ class FAOps:
                 sidecar = Path(metadata_path if metadata_path is not None
                                else str(Path(library_path).expanduser()) + ".json")
                 sidecar = sidecar.expanduser().resolve(strict=True)
-                self._validate(library, sidecar)
-                stamp = library.stat()
+                native = self._validate(library, sidecar)
+                files = [f for f in (library, native) if f is not None]
+
+                def stamps():
+                    return [(st.st_ino, st.st_size, st.st_mtime_ns) for st in (f.stat() for f in files)]
+                before = stamps()
 
                 def unchanged():
-                    now = library.stat()
-                    if (now.st_ino, now.st_size, now.st_mtime_ns) != \
-                            (stamp.st_ino, stamp.st_size, stamp.st_mtime_ns):
-                        raise CustomOpsError(f"{library} changed while it was being validated")
-                self._bind(library, unchanged)
+                    for f, a, b in zip(files, before, stamps()):
+                        if a != b:
+                            raise CustomOpsError(f"{f} changed while it was being validated")
+                self._bind(library, native, unchanged)
                 self._library, self._sidecar, self._error = library, sidecar, None
             except Exception as e:
                 self._error = str(e)
@@ -440,7 +482,8 @@ class FAOps:
 
     def load(self) -> "FAOps":
         """Development path: the in-tree library, compiled with hipcc when it is
-        missing and ``allow_jit`` is True."""
+        missing and ``allow_jit`` is True. The in-tree operator implementation is
+        opened only if it was built from the present sources for this PyTorch."""
         with _LOCK:
             if self._library is not None:
                 return self
@@ -453,7 +496,8 @@ class FAOps:
                 if not path.exists():
                     _build.build()
                 path = path.resolve(strict=True)
-                self._bind(path, lambda: None)
+                self._bind(path, Path(fa.OPS_PATH) if _build.ops_current(fa.OPS_PATH) else None,
+                           lambda: None)
                 self._library, self._sidecar, self._error = path, None, None
             except Exception as e:
                 self._error = str(e)

@@ -2775,13 +2775,15 @@ static bool exact_mask_weight(float scale) {
 // several row blocks re-read K and V and the splits are combined the fit is
 // least certain: there it has to win by a fifth. A variant or a split count set
 // by the caller selects among the tile kernels, except waves 1 or 2, which
-// force the streams (4 or 8 per workgroup).
+// force the streams (4 or 8 per workgroup), and except a split count above 1 that
+// is the streams' own choice: mi355_fa_num_splits' answer, given back, is the same
+// plan.
 static int pick_streams(const mi355_fa_params* p, const mi355_fa_variant& v, int cus, bool aligned,
                         int tile_waves, float tile_cost, int* splits) {
   const mi355_fa_variant none{};
   const bool forced = v.waves == 1 || v.waves == 2;
   const int fixed = p->num_splits > 0 ? p->num_splits : env_num_splits();
-  if (!forced && (fixed > 0 || memcmp(&v, &none, sizeof(v)) != 0)) return 0;
+  if (!forced && (fixed == 1 || memcmp(&v, &none, sizeof(v)) != 0)) return 0;
   if (p->seqlen_k < 1) return 0;
   // bf16 masks are added on the matrix core (see Attn::MMF); the 8-wave tile
   // kernel of 64-wide heads scales them by the fp32 1/scale where that is no bf16
@@ -2797,7 +2799,7 @@ static int pick_streams(const mi355_fa_params* p, const mi355_fa_variant& v, int
   const TileCost& tc = p->d == 64 ? kTileD64 : kTileD128;
   float limit = tc.c0 + tc.scale * tile_cost;
   if (!aligned) limit += tc.stage + tc.stage_m * ((float)p->b * p->seqlen_q * p->seqlen_k * 1e-6f);
-  int best = 0;
+  int best = 0, best_s = 0;
   float best_t = 0.f;
   for (int kg = 4; kg <= 8; kg += 4) {
     if (forced && kg != 4 * v.waves) continue;
@@ -2808,9 +2810,11 @@ static int pick_streams(const mi355_fa_params* p, const mi355_fa_variant& v, int
     for (int s = lo; s <= hi; ++s) {
       const float t = stream_cost(p, (int)std::min<int64_t>(blocks, 1 << 24), kg, s, cus);
       if (!forced && t >= (s > 1 && per > 1 ? 0.8f : 1.f) * limit) continue;
-      if (!best || t < best_t) { best = kg; best_t = t; *splits = s; }
+      if (!best || t < best_t) { best = kg; best_t = t; best_s = s; }
     }
   }
+  if (!best || (!forced && fixed > 0 && fixed != best_s)) return 0;
+  *splits = best_s;
   return best;
 }
 
@@ -2827,19 +2831,28 @@ static Plan make_plan(const mi355_fa_params* p, int cus, bool allow_stage = true
   const PlanCost& cm = p->d == 64 ? kCostD64 : kCostD128;
   int max_s = pl.num_n / 4 > 1 ? pl.num_n / 4 : 1;
   if (max_s > kMaxSplits) max_s = kMaxSplits;
-  float best = 0.f;
-  pl.waves = 0;
-  for (int w = 4; w <= 8; w += 4) {
-    if (w_fixed && w != w_fixed) continue;
-    for (int s = s_fixed > 0 ? s_fixed : 1; s <= (s_fixed > 0 ? s_fixed : max_s); ++s) {
-      const float c = plan_cost(cm, bh, p->seqlen_q, pl.num_n, p->d, w, s, cus, pl.pack);
-      if (pl.waves == 0 || c < best) { best = c; pl.waves = w; pl.splits = s; }
+  // cheapest workgroup size and split count (at `fixed` splits if > 0)
+  auto tile_plan = [&](int fixed, int* waves, int* splits) {
+    float best = 0.f;
+    *waves = 0;
+    for (int w = 4; w <= 8; w += 4) {
+      if (w_fixed && w != w_fixed) continue;
+      for (int s = fixed > 0 ? fixed : 1; s <= (fixed > 0 ? fixed : max_s); ++s) {
+        const float c = plan_cost(cm, bh, p->seqlen_q, pl.num_n, p->d, w, s, cus, pl.pack);
+        if (*waves == 0 || c < best) { best = c; *waves = w; *splits = s; }
+      }
     }
-  }
+    return best;
+  };
+  int auto_waves = 0, auto_splits = 0;
+  const float auto_cost = tile_plan(0, &auto_waves, &auto_splits);
+  pl.waves = auto_waves;
+  pl.splits = auto_splits;
+  if (s_fixed > 0) tile_plan(s_fixed, &pl.waves, &pl.splits);
   if (pl.splits < 1) pl.splits = 1;
   const bool mask_direct = ((uintptr_t)p->mask & 15) == 0 && (p->mask_batch_stride & 7) == 0 &&
                            (p->mask_row_stride & 7) == 0;
-  pl.ks = pick_streams(p, v, cus, mask_direct, pl.waves, best, &pl.splits);
+  pl.ks = pick_streams(p, v, cus, mask_direct, auto_waves, auto_cost, &pl.splits);
   const int s = pl.splits;
   pl.n_per_split = (s > 1) ? ceil_div(pl.num_n, s) : pl.num_n;
   if (s > 1) {

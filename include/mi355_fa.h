@@ -106,7 +106,8 @@ typedef struct mi355_fa_params {
   int32_t dtype;      /* MI355_FA_FP16 | MI355_FA_BF16 */
   float scale_softmax; /* 1/sqrt(d) in the reference op; any positive value allowed */
 
-  /* Split-KV: 0 = let the library plan it; >= 1 forces that many splits. */
+  /* Split-KV: 0 = let the library plan it; >= 1 forces that many splits, of a
+   * tile kernel (a count above 1 that is the plan's own gives the plan's kernel). */
   int32_t num_splits;
   /* Device workspace for split-KV partials, the fused split tail's ticket
    * words, and for masks with unaligned rows the live-tile map and an aligned

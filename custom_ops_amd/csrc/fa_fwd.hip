@@ -557,8 +557,16 @@ __device__ __forceinline__ rsrc_t mask_rsrc(CKParams& p, int b) {
 
 struct LiveProbe { u32x4 l, r; };
 
-// SAMPLE: 8 rows from the first to the last of the workgroup's `rows`, the
-// same for every wave (narrow_to_live's SHARE form).
+// A sample of the workgroup's `rows`, the same for every wave: 8 rows from the
+// first to the last. Byte offset of this lane's 16 bytes of it in tile 0.
+__device__ __forceinline__ uint32_t sample_offset(CKParams& p, const TileIdx& ti, int rows) {
+  const int lane = threadIdx.x & 63;
+  const int row = (lane >> 3) * (max(min(rows, p.sq - ti.m0), 1) - 1) / 7;
+  return ((uint32_t)(ti.m0 + row) * (uint32_t)p.m_rs + (uint32_t)(lane & 7) * 8u) * 2u;
+}
+
+// SAMPLE (narrow_to_live's SHARE form): the sample of the second tile and of the
+// last but one
 template <int NT, bool MAP = false, bool SCAN = true, bool LOCAL = false, bool SAMPLE = false>
 __device__ __forceinline__ LiveProbe live_probe(const TileIdx& ti, const KParams& pk, int rows = 0) {
   CKParams& p = kernarg_params(pk);
@@ -569,8 +577,13 @@ __device__ __forceinline__ LiveProbe live_probe(const TileIdx& ti, const KParams
   }
   const rsrc_t rm = mask_rsrc(p, ti.b);
   const int tid = threadIdx.x;
-  const int row = SAMPLE ? ((tid & 63) >> 3) * (max(min(rows, p.sq - ti.m0), 1) - 1) / 7 : tid >> 3;
-  const uint32_t rowoff = (uint32_t)(ti.m0 + row) * (uint32_t)p.m_rs + (uint32_t)(tid & 7) * 8u;
+  if constexpr (SAMPLE) {   // (launches that narrow have at least 4 tiles)
+    const uint32_t off = sample_offset(p, ti, rows);
+    pr.l = bload16(rm, off + kBN * 2u);
+    pr.r = bload16(rm, off + (uint32_t)(p.num_n - 2) * (kBN * 2));
+    return pr;
+  }
+  const uint32_t rowoff = (uint32_t)(ti.m0 + (tid >> 3)) * (uint32_t)p.m_rs + (uint32_t)(tid & 7) * 8u;
   // LOCAL: the ends of the workgroup's own split range, else of the key axis
   const int t0 = LOCAL ? ti.nb : 0, t1 = LOCAL ? max(ti.ne - 1, 0) : p.num_n - 1;
   pr.l = bload16(rm, (rowoff + (uint32_t)t0 * kBN) * 2u);
@@ -793,22 +806,25 @@ __device__ __forceinline__ bool range_from_map_wave(TileIdx& ti, CKParams& p, in
 // Shared scan (unsplit ping-pong launches, whose head groups all need the live
 // range of the same rows): instead of each scanning the row block's dead tiles
 // ([4,16,2048,2048] causal: 115 MB of mask per round through the L2s, 17 µs),
-// the sg head groups of a row block that run on one XCD at once divide it:
-// the j-th tests tiles j, j + sg, j + 2·sg, .., publishes the verdicts in its
-// own word, and reads the others' words. That shape: 122 µs with every
-// workgroup scanning, 98-101 shared (131 with no narrowing; all 16 heads, on two
+// the sg head groups of a row block that run on one XCD at once divide the tiles
+// outside the ones known to be live (`outside` of them: 0 .. left - 1 and
+// right + 1 on): the j-th tests the j-th, (j + sg)-th, .. of them, publishes the
+// verdicts in its own word, and reads the others' words. That shape: 114 µs with every
+// workgroup scanning, 97 shared (127 with no narrowing; all 16 heads, on two
 // XCDs, start apart: 109).
 // A word is a 48-bit launch tag above 16 verdict bits, written and read at
 // device scope (sc1), with one writer, who clears it before it ends: a
 // replayed graph launch, which carries the same tag, finds no word of the
 // replay before. Nothing depends on another workgroup: after a bounded number
-// of polls (head groups that are not running yet) the caller scans by itself.
-// Returns whether the words gave the range [lo, hi] (hi < lo: no visible
-// entry). red: 2·NT/64 words of LDS.
+// of polls (head groups that are not running yet, or gone), about as long as its
+// own scan takes, the caller scans by itself.
+// Returns whether the words gave the outermost live ones [lo, hi] (lo = 2^31 - 1,
+// hi = -1: none). red: 2·NT/64 words of LDS.
 template <bool BF16, int NT>
-__device__ __forceinline__ bool share_scan(const TileIdx& ti, int rows, int& lo, int& hi, uint32_t* red) {
+__device__ __forceinline__ bool share_scan(const TileIdx& ti, int rows, int left, int right, int outside,
+                                           int& lo, int& hi, uint32_t* red) {
   CKParams& p = *reload_params();
-  const int sg = p.scan_group, nn = p.num_n, hg = (ti.h / p.pack) % sg;   // place in the group
+  const int sg = p.scan_group, hg = (ti.h / p.pack) % sg;   // place in the group
   const int nr = min(rows, p.sq - ti.m0);
   if (nr <= 0) return false;
   const int tid = threadIdx.x;
@@ -823,23 +839,25 @@ __device__ __forceinline__ bool share_scan(const TileIdx& ti, int rows, int& lo,
     off[j] = c < cpt ? ((uint32_t)(ti.m0 + (c >> 3)) * (uint32_t)p.m_rs + (uint32_t)(c & 7) * 8u) * 2u : 0xfffffff0u;
   }
   const int c0 = (tid & 7) * 8;
-  uint32_t bits = 0u;                  // bit k: tile hg + k·sg holds a visible entry
-  for (int k = 0; hg + k * sg < nn; k += kPer) {
+  auto tile = [&](int c) { return c < left ? c : c - left + right + 1; };
+  uint32_t bits = 0u;                  // bit k: outside tile hg + k·sg holds a visible entry
+  for (int k = 0; hg + k * sg < outside; k += kPer) {
     u32x4 v[kPer][kJ];
 #pragma unroll
     for (int u = 0; u < kPer; ++u)
 #pragma unroll
       for (int j = 0; j < kJ; ++j) {
-        const int t = hg + (k + u) * sg;
-        v[u][j] = bload16(rm, t < nn && off[j] != 0xfffffff0u ? off[j] + (uint32_t)t * (kBN * 2) : 0xfffffff0u);
+        const int c = hg + (k + u) * sg;
+        v[u][j] = bload16(rm, c < outside && off[j] != 0xfffffff0u ? off[j] + (uint32_t)tile(c) * (kBN * 2)
+                                                                   : 0xfffffff0u);
       }
 #pragma unroll
     for (int u = 0; u < kPer; ++u)
 #pragma unroll
       for (int j = 0; j < kJ; ++j) {
-        const int t = hg + (k + u) * sg;
-        const bool in = t < nn && off[j] != 0xfffffff0u;
-        bits |= (in & live8<BF16>(v[u][j], t * kBN + c0, p.sk)) ? 1u << (k + u) : 0u;
+        const int c = hg + (k + u) * sg;
+        const bool in = c < outside && off[j] != 0xfffffff0u;
+        bits |= (in & live8<BF16>(v[u][j], tile(c) * kBN + c0, p.sk)) ? 1u << (k + u) : 0u;
       }
   }
   bits = wave_or(bits);
@@ -855,14 +873,17 @@ __device__ __forceinline__ bool share_scan(const TileIdx& ti, int rows, int& lo,
     if (tid == 0)
       __hip_atomic_store(slots + hg, tag | mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     int found = 0, l = 0x7fffffff, h = -1;
-    constexpr int kPolls = 30;         // about 1 µs each
-    for (int it = 0; it < kPolls && !found; ++it) {
+    // about 1 µs each. As long as the caller's own scan takes on a busy chip, and
+    // no less: groups that straddle a round catch up by it ([8,7,2048,2048] causal
+    // 83 µs, with half as many polls 104)
+    const int polls = 4 + outside;
+    for (int it = 0; it < polls && !found; ++it) {
       const unsigned long long w = tid == hg ? tag | mine
           : tid < sg ? __hip_atomic_load(slots + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : tag;
       if (__builtin_amdgcn_ballot_w64((w >> 16) != p.tag) == 0) {
         found = 1;
         const uint32_t x = (uint32_t)(w & 0xffffu);
-        if (x) { l = tid + __builtin_ctz(x) * sg; h = tid + (31 - __builtin_clz(x)) * sg; }
+        if (x) { l = tile(tid + __builtin_ctz(x) * sg); h = tile(tid + (31 - __builtin_clz(x)) * sg); }
       } else {
         __builtin_amdgcn_s_sleep(16);
       }
@@ -893,8 +914,15 @@ __device__ __forceinline__ void share_clear(const TileIdx& ti, int rows) {
 // Scanning the whole axis to re-partition the live range (the assembly
 // loops) reads a sparse mask's dead part once per split and head: a top-left
 // causal [1,16,16,128,32768] took 357 µs that way on 16 splits.
-// SHARE: through share_scan first, when the launch has the words (`shared` is
-// set when the workgroup published its own, which it then has to clear).
+// SHARE: an end whose second tile shows a visible entry in the sample stays
+// nominal (one dead tile, 1 µs, is cheaper than the look for it). Else samples
+// across the key axis bound the range from inside: at most kNear tiles away from
+// both ends the workgroup scans by itself, further in the scan comes through
+// share_scan, if the launch has the words (`shared` is set when the workgroup
+// published its own, which it then has to clear). Looking through all tiles, and
+// together, whenever the first or the last one was dead ran keys padded by one
+// tile at 150 µs on [4,16,2048,2048] (now 133) and 284 on Sk 4096 (244), slower
+// than with no look at all (132 and 242); causal at Sk 4096 224 -> 207.
 template <bool BF16, int NT, int BMAX, int J, bool REUSE, bool MAP = false, bool SCAN = true, bool LOCAL = false,
           bool SHARE = false>
 __device__ __forceinline__ bool narrow_to_live(TileIdx& ti, const KParams& pk, int rows, const LiveProbe& pr,
@@ -917,11 +945,14 @@ __device__ __forceinline__ bool narrow_to_live(TileIdx& ti, const KParams& pk, i
   if (LOCAL && first > last) return false;   // an empty share stays empty
   // the probe's verdict: tile first / tile last live in the chunks it read
   bool lb, rb;
+  auto sampled = [&](u32x4 v, int t) {
+    return __builtin_amdgcn_ballot_w64(live8<BF16>(v, t * kBN + (tid & 7) * 8, p.sk)) != 0;
+  };
   if constexpr (SHARE) {
     // a sample of the rows, the same for every wave: a live entry in it settles
     // its end without an exchange (a miss only means the scan, which decides)
-    lb = __builtin_amdgcn_ballot_w64(live8<BF16>(pr.l, first * kBN + (tid & 7) * 8, p.sk)) != 0;
-    rb = __builtin_amdgcn_ballot_w64(live8<BF16>(pr.r, last * kBN + (tid & 7) * 8, p.sk)) != 0;
+    lb = sampled(pr.l, first + 1);
+    rb = sampled(pr.r, last - 1);
   } else {
     lb = (tid < nr * 8) & live8<BF16>(pr.l, first * kBN + (tid & 7) * 8, p.sk);
     rb = (tid < nr * 8) & live8<BF16>(pr.r, last * kBN + (tid & 7) * 8, p.sk);
@@ -931,12 +962,38 @@ __device__ __forceinline__ bool narrow_to_live(TileIdx& ti, const KParams& pk, i
     if constexpr (!SHARE) __syncthreads();   // every wave has read `red` before any DMA lands
     return false;
   }
-  int lo = lb ? first : -1, hi = rb ? last : -1;
   if constexpr (SHARE) {
-    if (p.scan_slots) {
+    // (each wave one of 8 places; 4 tiles are one step of the scan below)
+    constexpr int kNear = 4;
+    static_assert(NT == 512, "8 waves, 8 places");
+    const int w = tid >> 6, q = nn / 4, in = (w & 3) == 0 ? 0 : (w & 3) == 1 ? min(kNear, q) : (w & 3) == 2 ? q : nn / 2;
+    const int at = w < 4 ? in : last - in;
+    const u32x4 smp = bload16(mask_rsrc(p, ti.b), sample_offset(p, ti, rows) + (uint32_t)at * (kBN * 2));
+    int* const found = reinterpret_cast<int*>(red + 64);
+    found[w] = sampled(smp, at) ? at : -1;
+    __syncthreads();
+    // the outermost tiles known to be live (none: nn, -1)
+    int left = nn, right = -1;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int f = found[i];
+      left = f < 0 ? left : min(left, f);
+      right = max(right, f);
+    }
+    left = __builtin_amdgcn_readfirstlane(left);
+    right = __builtin_amdgcn_readfirstlane(right);
+    lb = lb || left == 0;
+    rb = rb || right == last;
+    if (lb && rb) return false;
+    if (lb) { left = 0; right = max(right, 0); }
+    if (rb) { right = last; left = min(left, last); }
+    if (p.scan_slots && (left > kNear || last - right > kNear)) {
       *shared = true;
       int l, h;
-      if (share_scan<BF16, NT>(ti, rows, l, h, red)) {
+      const int from = left == nn ? last : right;   // (none known: all tiles, as the left ones)
+      if (share_scan<BF16, NT>(ti, rows, left, from, left + last - from, l, h, red)) {
+        l = min(l, left);
+        h = max(h, right);
         if (h < l) { l = 0; h = -1; }
         ti.nb = l;
         ti.ne = h + 1;
@@ -944,6 +1001,7 @@ __device__ __forceinline__ bool narrow_to_live(TileIdx& ti, const KParams& pk, i
       }
     }
   }
+  int lo = lb ? first : -1, hi = rb ? last : -1;
   constexpr int kRounds = (8 * BMAX + J * NT - 1) / (J * NT);   // rounds that cover one whole tile
   constexpr int NL = kRounds * J;
   const int cpt = nr * 8;                  // 16-byte chunks per tile of these rows
@@ -2947,7 +3005,8 @@ static Plan make_plan(const mi355_fa_params* p, int cus, bool allow_stage = true
   // Unsplit ping-pong launches of more than one round whose workgroups probe
   // and scan (aligned mask rows), in an order that runs a row block's head
   // groups together (m-blocks fastest, their waits ran [4,16,2048,2048] causal
-  // at 162 µs instead of 102): words for the shared scan, 16 tiles per word
+  // at 162 µs instead of 102): words for the shared scan, 16 tiles per word, for
+  // groups that one XCD's CUs can run together
   {
     const int ng = p->h / pl.pack;
     const int64_t total = (int64_t)p->b * ng * pl.num_m;
@@ -2955,7 +3014,7 @@ static Plan make_plan(const mi355_fa_params* p, int cus, bool allow_stage = true
     const int sg = pl.head_major == 3 && pl.sub < ng ? pl.sub : ng;
     if (s == 1 && pl.waves == 8 && mask_direct && pl.head_major != 0 && !pl.live_map && pl.live != 0 && pl.loop == 3 && p->d == 128 &&
         p->dtype == MI355_FA_BF16 && p->scale_softmax < 0.99f && pl.num_n >= 4 && total > cus && ng % sg == 0 &&
-        sg >= 4 && sg <= 64 && pl.num_n <= 16 * sg) {
+        sg >= 4 && sg <= cus / 8 && pl.num_n <= 16 * sg) {
       pl.scan_bytes = ((size_t)total * 8 + 255) & ~(size_t)255;
       pl.scan_group = sg;
     }

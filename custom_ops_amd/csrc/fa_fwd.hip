@@ -2695,9 +2695,9 @@ struct Plan {
   // rows: 3 = ping-pong (bf16; fp16 runs the 32-row loop), 1 = 32-row loop,
   // 2 = 64-row loop, 0 = the compiled kernel.
   int loop;
-  // Live-range narrowing: 2 = the default policy (on for split launches and
-  // for the compiled kernel, off for unsplit launches of the assembly loops),
-  // 1 = on everywhere, 0 = off.
+  // Live-range narrowing: 2 = the default policy (on for split launches, for
+  // the compiled kernel and for the ping-pong loop, off for unsplit launches of
+  // the 32- and 64-row loops), 1 = on everywhere, 0 = off.
   int live;
   int mask_mfma_off;   // the compiled kernel widens bf16 masks on the VALU
   int kv_nt;           // every K/V tile is read by one workgroup: non-temporal loads
@@ -2826,16 +2826,20 @@ static bool exact_mask_weight(float scale) {
 }
 
 // Whether the key-stream kernel runs this call, with how many streams per
-// workgroup (4 or 8; 0: a tile kernel) and splits: where the models put it
-// below the tile plan's `tile_cost`. Over those 370 shapes the choice runs 1.34
-// times as fast as the tile plans alone (geometric mean; the best choice for
-// each shape 1.36), never over 8 % slower. Every stream keeps two tiles. Where
-// several row blocks re-read K and V and the splits are combined the fit is
-// least certain: there it has to win by a fifth. A variant or a split count set
-// by the caller selects among the tile kernels, except waves 1 or 2, which
-// force the streams (4 or 8 per workgroup), and except a split count above 1 that
-// is the streams' own choice: mi355_fa_num_splits' answer, given back, is the same
-// plan.
+// workgroup (4 or 8; 0: a tile kernel) and splits: where the models put it below
+// the tile plan's `tile_cost` by enough to be sure of it. The lines come from 2400
+// calls of all kinds of masks, aligned or not. Taken for any gain promised (a fifth
+// where it splits and several row blocks re-read K and V), 1926 calls ran 1.529
+// times as fast as under the tile plans (geometric mean), but 51 of them below 0.97:
+// nearly all 128-wide heads promised less than 15 %, on grids of more than one
+// round ([2,8,2205,2205] 88 µs against 64, [3,8/1,1604,1604] 67 against 54) or with
+// one or two tiles per stream ([4,32/16,96,96] 8.7 against 8.0). Those have to
+// promise 25 and 15 %; others 5 %, but for 64-wide heads with unaligned masks, which
+// gain up to the line: 1.530, 6 calls below 0.97, none below 0.85. Every stream keeps
+// two tiles. A variant or a split count set by the caller selects among the tile kernels, except
+// waves 1 or 2, which force the streams (4 or 8 per workgroup), and except a split
+// count above 1 that is the streams' own choice: mi355_fa_num_splits' answer, given
+// back, is the same plan.
 static int pick_streams(const mi355_fa_params* p, const mi355_fa_variant& v, int cus, bool aligned,
                         int tile_waves, float tile_cost, int* splits) {
   const mi355_fa_variant none{};
@@ -2867,7 +2871,14 @@ static int pick_streams(const mi355_fa_params* p, const mi355_fa_variant& v, int
     const int lo = forced && fixed > 0 ? std::min(fixed, kMaxSplits) : 1, hi = forced && fixed > 0 ? lo : max_s;
     for (int s = lo; s <= hi; ++s) {
       const float t = stream_cost(p, (int)std::min<int64_t>(blocks, 1 << 24), kg, s, cus);
-      if (!forced && t >= (s > 1 && per > 1 ? 0.8f : 1.f) * limit) continue;
+      // how far below the tile plan
+      const float rounds = (float)blocks * (float)s / (float)(cus * (8 / kg));
+      float line = 0.95f;
+      if (s > 1 && per > 1) line = 0.8f;
+      else if (p->d == 64 && !aligned) line = 1.f;
+      else if (p->d == 128 && rounds > 1.f) line = 0.75f;
+      else if (p->d == 128 && ceil_div(ntile, s * kg) <= 2) line = 0.85f;
+      if (!forced && t >= line * limit) continue;
       if (!best || t < best_t) { best = kg; best_t = t; best_s = s; }
     }
   }

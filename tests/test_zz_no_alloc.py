@@ -60,8 +60,8 @@ def test_noalloc_matches_workspace_entry_two_calls(dtype):
         # the second is smaller and reuses it
         (1, 16, 16, 128, 16384, 128, 16, 11),
         (1, 4, 2, 100, 3001, 64, 5, 12),
-        # unsplit, unaligned mask rows: the staged mask (and no map: the
-        # assembly loop does not narrow unsplit launches) in the array
+        # unsplit, unaligned mask rows: the staged mask (with the map of its live
+        # tiles, which the bf16 loop reads) in the array
         (2, 4, 4, 300, 777, 128, 1, 13),
     ]
     for b, h, hk, sq, sk, d, splits, seed in cases:

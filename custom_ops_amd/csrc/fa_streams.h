@@ -427,11 +427,9 @@ void fa_fwd_kernel_ks(const KParams p) {
 #pragma unroll
       for (int i = 0; i < kLoads; ++i)
         *reinterpret_cast<u32x4*>(st + i * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
-    };
-    if (p.sk % kTS != 0) {
-      clear(sV);
       wait_lds();
-    }
+    };
+    if (p.sk % kTS != 0) clear(sV);
     // The first tile's K and V are loaded whatever its mask holds. With one
     // buffer the second tile's mask leaves when the first's has been read.
     // Where it is all -inf they are cleared: NaN in them (rows of a cache that
@@ -451,7 +449,6 @@ void fa_fwd_kernel_ks(const KParams p) {
     if (__builtin_expect(!M::any(mraw), 0)) {
       clear(sK);
       clear(sV);
-      wait_lds();
     }
 
     bool live = true;
